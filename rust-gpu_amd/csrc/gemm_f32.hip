@@ -1,0 +1,73 @@
+// gemm_f32.hip — launches of the one-launch f32-operand GEMM (gemm_f32.h) for the Ignis matmul
+// (src/ignis/ops/bf16_matmul.rs:33-316).
+#include "gemm_f32.h"
+
+#include <string.h>
+
+#include "t0mi_ctx.h"
+
+namespace t0mi {
+
+namespace {
+
+template <int I, bool AK, bool BKM>
+void launch(const GemmF32Params& p, uint32_t grid, hipStream_t s) {
+  constexpr int BM = kF32Tiles[I].bm, BN = kF32Tiles[I].bn, G = kF32Tiles[I].groups;
+  constexpr int WM = I == 0 ? 1 : I == 3 ? 4 : 2, WN = I < 2 ? 1 : I == 4 ? 4 : 2;  // 8 waves with G
+  hipLaunchKernelGGL((gemm_f32_kernel<BM, BN, kF32Bk, WM, WN, G, 2, AK, BKM>), dim3(grid), dim3(WM * WN * G * 64), 0,
+                     s, p);
+}
+
+template <bool AK, bool BKM>
+void launch_tile(int tile, const GemmF32Params& p, uint32_t grid, hipStream_t s) {
+  switch (tile) {
+    case 0: launch<0, AK, BKM>(p, grid, s); break;
+    case 1: launch<1, AK, BKM>(p, grid, s); break;
+    case 2: launch<2, AK, BKM>(p, grid, s); break;
+    case 3: launch<3, AK, BKM>(p, grid, s); break;
+    default: launch<4, AK, BKM>(p, grid, s); break;
+  }
+}
+
+bool overlap(uint64_t a, uint64_t an, uint64_t b, uint64_t bn) { return a < b + bn && b < a + an; }
+
+}  // namespace
+
+int run_gemm_f32(t0mi_ctx* ctx, int mode, uint64_t a, uint64_t b, uint64_t y, uint32_t m, uint32_t n, uint32_t k) {
+  if (ctx->null_backend) return 1;
+  const F32Plan plan = f32_plan(mode, m, n, k, (uint32_t)ctx->cu_count, ctx->xk_nx > 0);
+  if (plan.tile < 0) return 1;
+  const uint64_t a_bytes = (uint64_t)m * k * 4, b_bytes = (uint64_t)k * n * 4, y_bytes = (uint64_t)m * n * 4;
+  // Y over an operand: the conversion passes read both operands whole before Y is written.
+  if (overlap(a, a_bytes, y, y_bytes) || overlap(b, b_bytes, y, y_bytes)) return 1;
+  GemmF32Params p;
+  memset(&p, 0, sizeof p);
+  p.a = (const float*)a;
+  p.b = (const float*)b;
+  p.y = (float*)y;
+  p.M = m;
+  p.N = n;
+  p.K = k;
+  p.lda = f32_a_kmajor(mode) ? m : k;
+  p.ldb = f32_b_kmajor(mode) ? n : k;
+  p.a_bytes = (uint32_t)a_bytes;
+  p.b_bytes = (uint32_t)b_bytes;
+  p.tiles_m = plan.tiles_m;
+  p.tiles_n = plan.tiles_n;
+  p.pieces = plan.pieces;
+  uint32_t grid = plan.tiles_m * plan.tiles_n;
+  if (plan.pieces > 1) {
+    bool ok = false;
+    if (xk_prepare(ctx, grid, kF32SlotBytes, &p.x, &ok) != T0MI_OK || !ok) return 1;
+    grid = (grid + p.x.nx - 1) / p.x.nx * p.x.nx * plan.pieces;
+  }
+  switch (mode) {
+    case F32_FORWARD: launch_tile<false, true>(plan.tile, p, grid, ctx->stream); break;
+    case F32_DATA: launch_tile<false, false>(plan.tile, p, grid, ctx->stream); break;
+    default: launch_tile<true, true>(plan.tile, p, grid, ctx->stream); break;
+  }
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? T0MI_OK : set_error(T0MI_ERR_HIP, "f32 GEMM launch: %s", hipGetErrorString(e));
+}
+
+}  // namespace t0mi

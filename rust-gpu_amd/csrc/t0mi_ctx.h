@@ -198,4 +198,9 @@ const char* persistent_route(const t0mi_gemm_config& cfg, uint32_t m, uint32_t n
 int run_gemm_persistent(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e, uint64_t x,
                         uint64_t b, uint64_t y, uint64_t bias, uint32_t m, uint32_t n, uint32_t k,
                         const EpiChain& epi);
+// Y[m,n] = bf16(A) . bf16(B) over K = k with f32 operands in one launch (gemm_f32.h); `mode` is a
+// F32Mode.  Returns 1, launching nothing, where the conversion passes and the bf16 GEMM are the
+// route (f32_plan, operands that overlap Y, an exchange buffer that may not grow now).
+// Asynchronous.
+int run_gemm_f32(t0mi_ctx* ctx, int mode, uint64_t a, uint64_t b, uint64_t y, uint32_t m, uint32_t n, uint32_t k);
 }  // namespace t0mi

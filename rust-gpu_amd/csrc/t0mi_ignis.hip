@@ -5,15 +5,17 @@
 // The reference reads its f32 operands back to the host, converts them to bf16
 // (round to nearest even, bf16_matmul.rs:372), transposes W, pads every
 // dimension to the tile size, uploads, runs the NT kernel and unpads the f32
-// result with a second kernel.  Here one HBM-bound kernel converts (and, for
-// the weight gradient's X^T operand, transposes through LDS) into a
-// library-owned bf16 buffer; the GEMM takes NN or NT natively and masks ragged
+// result with a second kernel.  Here small and mid-sized products run as one
+// launch on the f32 operands (gemm_f32.h).  For large ones an HBM-bound kernel
+// converts (and, for the weight gradient's X^T operand, transposes through LDS)
+// into a library-owned bf16 buffer once; the GEMM takes NN or NT natively and masks ragged
 // tiles, so padding is needed only to give K and N the 8-element (16-byte)
 // row granularity of the GEMM's loads, and only then is the result unpadded.
 #include <string.h>
 
 #include <algorithm>
 
+#include "gemm_f32_plan.h"
 #include "t0mi_ctx.h"
 
 using namespace t0mi;
@@ -227,6 +229,7 @@ extern "C" int t0mi_matmul_f32(t0mi_ctx* ctx, uint64_t x, uint64_t w, uint64_t y
   if (rc) return rc;
   T0MI_SUBMIT_GUARD(ctx);
   if (m == 0 || n == 0) return T0MI_OK;
+  if ((rc = run_gemm_f32(ctx, F32_FORWARD, x, w, y, m, n, k)) <= 0) return rc;
   const uint32_t kp = up8(k), np = up8(n);
   const size_t xa = align256((size_t)m * kp * 2), wb = align256((size_t)kp * np * 2);
   const size_t pad = np != n ? (size_t)m * np * 4 : 0;
@@ -263,6 +266,7 @@ extern "C" int t0mi_matmul_backward_data(t0mi_ctx* ctx, uint64_t dy, uint64_t w,
   if (rc) return rc;
   T0MI_SUBMIT_GUARD(ctx);
   if (m == 0 || k == 0) return T0MI_OK;
+  if ((rc = run_gemm_f32(ctx, F32_DATA, dy, w, dx, m, k, n)) <= 0) return rc;
   const uint32_t cp = up8(n), op = up8(k);  // contraction n, output columns k
   const size_t da = align256((size_t)m * cp * 2), wb = align256((size_t)op * cp * 2);
   const size_t pad = op != k ? (size_t)m * op * 4 : 0;
@@ -283,6 +287,7 @@ extern "C" int t0mi_matmul_backward_weight(t0mi_ctx* ctx, uint64_t x, uint64_t d
   if (rc) return rc;
   T0MI_SUBMIT_GUARD(ctx);
   if (k == 0 || n == 0) return T0MI_OK;
+  if ((rc = run_gemm_f32(ctx, F32_WEIGHT, x, dy, dw, k, n, m)) <= 0) return rc;
   const uint32_t cp = up8(m), np = up8(n);  // contraction m, output columns n
   const size_t xa = align256((size_t)k * cp * 2), db = align256((size_t)cp * np * 2);
   const size_t pad = np != n ? (size_t)k * np * 4 : 0;
