@@ -2,6 +2,9 @@
 // conversion passes plus the bf16 GEMM take it; and the kernel's global index maps.  Plain
 // arithmetic (no HIP), also compiled into the CPU test of both (tests/gemm_f32_plan_sim.cpp).
 #pragma once
+#if defined(__HIPCC__)
+#include <hip/hip_runtime.h>
+#endif
 #include <stdint.h>
 
 #include "index_maps.h"
