@@ -787,6 +787,10 @@ static float rd_f32(const uint8_t* p) {
   return f;
 }
 
+static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e,
+                         uint64_t x, uint64_t b, uint64_t y, uint64_t bias, uint32_t m, uint32_t n, uint32_t k,
+                         const EpiChain& chain);
+
 // Dispatch of a lowered TileGemm with its own kernarg layout (tile_ir.rs:4570-4637
 // plus the epilogue arguments declared at :1014-1027).
 static int dispatch_tile(t0mi_ctx* ctx, const t0mi_kernel* k, const uint32_t grid[3], const uint8_t* ka) {
@@ -825,7 +829,7 @@ static int dispatch_tile(t0mi_ctx* ctx, const t0mi_kernel* k, const uint32_t gri
     return run_gemm_persistent(ctx, k->cfg, k->gemm, x, wt, y, bias, M, N, K, chain);
   if (sk == 1 || yss == 0)
     // One output plane: split-K partitions are summed by the library.
-    return run_gemm(ctx, k->cfg, k->gemm, x, wt, y, bias, M, N, K, chain);
+    return run_tile_gemm(ctx, s, k->cfg, k->gemm, x, wt, y, bias, M, N, K, chain);
   // Caller-provided partial planes (gemm_gen convention): partition p writes
   // the raw f32 sum of its K range at Y + p * y_split_stride; no epilogue.
   if (K % 8 || N % 8 || (K / sk) % 8)
@@ -1163,6 +1167,29 @@ extern "C" int t0mi_auto_gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t 
 
 // ------------------------------------------------------------ tile_ir GEMM ----
 
+// Y = epi(X . B) of a one-shot spec into one plane.  A spec without split-K leaves the schedule
+// open, and its tile is one of an RDNA part's (64 x 64 x 16 on one wave, say), so the schedule that
+// auto_select ranks first for the shape runs under the spec's name, kernargs and grid, as for the
+// persistent presets (1000 x 2752 x 2056 NT, bias + GELU, bf16 out, tile_auto_select's 64x64 k16: TILE_US_BEFORE
+// us on its own tile, TILE_US_AFTER so).  The spec's tile remains for specs that name their split-K, for
+// calls whose arguments are refused (it reports them), and where the schedule's split-K planes would
+// need workspace that may not grow now (a capture, or live graphs holding its address).
+static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e,
+                         uint64_t x, uint64_t b, uint64_t y, uint64_t bias, uint32_t m, uint32_t n, uint32_t k,
+                         const EpiChain& chain) {
+  const bool valid = m && n && k && k % 8 == 0 && n % 8 == 0 && !((x | b | y) & 15) && !(bias & 3) &&
+                     !(chain_uses(chain, EOP_BIAS) && !bias);
+  AutoPlan pl;
+  if (tile_split_k(s) == 1 && valid &&
+      cached_auto_plan(m, n, k, cfg.transpose, cfg.out_dtype, (uint32_t)ctx->cu_count, &pl)) {
+    const uint32_t sk_h = split_k_of(pl.head), sk_t = pl.n1 < n ? split_k_of(pl.tail) : 1;
+    const size_t need = std::max(sk_h > 1 ? (size_t)m * pl.n1 * 4 * sk_h : 0, sk_t > 1 ? (size_t)m * (n - pl.n1) * 4 * sk_t : 0);
+    if (need <= ctx->ws_bytes || (ctx->live_graphs.load() == 0 && refuse_if_capturing(ctx, "growth") == T0MI_OK))
+      return run_gemm_auto(ctx, cfg.transpose, x, b, y, m, n, k, cfg.out_dtype, bias, &chain);
+  }
+  return run_gemm(ctx, cfg, e, x, b, y, bias, m, n, k, chain);
+}
+
 extern "C" int t0mi_tile_kernel_get(t0mi_ctx* ctx, const t0mi_tile_spec* s, t0mi_kernel** out) {
   if (!ctx || !s || !out) return set_error(T0MI_ERR_INVALID, "null argument");
   EpiChain chain;
@@ -1218,5 +1245,5 @@ extern "C" int t0mi_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec* s, uint64_t x
   chain.lo = clamp_min;
   chain.hi = clamp_max;
   if (s->persistent) return run_gemm_persistent(ctx, cfg, e, x, wt, y, bias, m, n, k, chain);
-  return run_gemm(ctx, cfg, e, x, wt, y, bias, m, n, k, chain);
+  return run_tile_gemm(ctx, *s, cfg, e, x, wt, y, bias, m, n, k, chain);
 }
