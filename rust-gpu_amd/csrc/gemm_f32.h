@@ -54,9 +54,6 @@ struct GemmF32Params {
   XcdExchange x;
 };
 
-// 16 bytes at any 4-byte aligned address.
-typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
-
 // One operand's tile: ROWS rows (or columns) of the product by BK of K, loaded by NT threads as
 // NP 16-byte pieces each; KM: K-major.
 template <int ROWS_, int BK_, int NT, bool KM_>

@@ -159,22 +159,14 @@ __global__ __launch_bounds__(PD_WAVES * 64) void gemm_persistent_decode_kernel(G
         f32x4 s = red[0][h][src];
 #pragma unroll
         for (int w = 1; w < PD_WAVES; ++w) s += red[w][h][src];
-        float v0 = s.x, v1 = s.y, v2 = s.z, v3 = s.w;
-        if (p.epi.n) {
-          f32x4 bv = {0.0f, 0.0f, 0.0f, 0.0f};
-          if (p.bias) bv = f32x4{p.bias[n], p.bias[n + 1], p.bias[n + 2], p.bias[n + 3]};
-          v0 = epi_apply(v0, bv.x, p.epi);
-          v1 = epi_apply(v1, bv.y, p.epi);
-          v2 = epi_apply(v2, bv.z, p.epi);
-          v3 = epi_apply(v3, bv.w, p.epi);
-        }
+        if (p.epi.n) s = epi_apply4(s, p.bias, (uint32_t)n, p.epi);
         if (p.out_bf16) {
           u32x2 o;
-          o.x = pack_bf16x2(v0, v1);
-          o.y = pack_bf16x2(v2, v3);
+          o.x = pack_bf16x2(s.x, s.y);
+          o.y = pack_bf16x2(s.z, s.w);
           *(u32x2*)((uint16_t*)p.y + (size_t)m * p.ldy + n) = o;
         } else {
-          *(f32x4*)((float*)p.y + (size_t)m * p.ldy + n) = f32x4{v0, v1, v2, v3};
+          *(f32x4*)((float*)p.y + (size_t)m * p.ldy + n) = s;
         }
       }
     }

@@ -369,19 +369,24 @@ __global__ __launch_bounds__(512) void gemm_bf16_pingpong_kernel(GemmParams p) {
     else
       store_tile_bf16_staged<FM, FN>(p, acc, (char*)smem + wave * 16384, ybase, row0, col0, lane);
   } else {
-    static_for<FM>([&](auto fmc) {
-      constexpr int fm = decltype(fmc)::value;
-      const int m = row0 + fm * MB + lrow;
-      if (m < (int)p.M) {
-        static_for<FN>([&](auto fnc) {
-          constexpr int fn = decltype(fnc)::value;
-          if constexpr (X16)
-            store_block16(p, acc[fn][fm], ybase, m, col0 + fn * 16 + lgrp * 4, partial_plane);
-          else
-            store_block(p, acc[fn][fm], ybase, m, col0 + fn * 32 + lgrp * 4, partial_plane);
-        });
-      }
-    });
+    if constexpr (X16) {
+      BiasCols<4> bias;
+      bias.load(p, col0 + lgrp * 4, 16);
+      static_for<FM>([&](auto fmc) {
+        constexpr int fm = decltype(fmc)::value;
+        const int m = row0 + fm * MB + lrow;
+        if (m < (int)p.M) {
+          float v[16];
+          epi_row16<FM>(p, acc, fm, partial_plane, bias, v);
+          static_for<FN>([&](auto fnc) {
+            constexpr int fn = decltype(fnc)::value;
+            store_block16(p, v + fn * 4, ybase, m, col0 + fn * 16 + lgrp * 4, partial_plane);
+          });
+        }
+      });
+    } else {
+      store_tile_direct<FM, FN>(p, acc, ybase, row0, col0, lane, partial_plane);
+    }
   }
 }
 

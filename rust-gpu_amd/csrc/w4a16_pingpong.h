@@ -386,16 +386,7 @@ __global__ __launch_bounds__(512) void w4a16_pingpong_kernel(W4PPParams q) {
   if (!partial_plane && p.out_bf16 && m0 + 256 <= (int)p.M && n0 + 256 <= (int)p.N && ((uintptr_t)p.y & 15) == 0) {
     store_tile_bf16_staged<FM, FN>(p, acc, (char*)smem + wave * 16384, ybase, row0, col0, lane);
   } else {
-    static_for<FM>([&](auto fmc) {
-      constexpr int fm = decltype(fmc)::value;
-      const int m = row0 + fm * 32 + lrow;
-      if (m < (int)p.M) {
-        static_for<FN>([&](auto fnc) {
-          constexpr int fn = decltype(fnc)::value;
-          store_block(p, acc[fn][fm], ybase, m, col0 + fn * 32 + lhalf * 4, partial_plane);
-        });
-      }
-    });
+    store_tile_direct<FM, FN>(p, acc, ybase, row0, col0, lane, partial_plane);
   }
 }
 
