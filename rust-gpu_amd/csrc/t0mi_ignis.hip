@@ -104,47 +104,80 @@ __global__ __launch_bounds__(256) void unpad_f32_kernel(const float* __restrict_
   }
 }
 
-// GPTQ packed [N][K/2] bytes viewed as u32 [N][K/8] -> qweight u32 [K/8][N]:
-// the little-endian word of GPTQ bytes 4kk..4kk+3 of row n holds elements
-// 8kk..8kk+7 of that row at bits 4e (element 2i = low nibble of byte i), which
-// is word (kk, n) of the W4A16 layout.  64x64 tiles through LDS.
-__global__ __launch_bounds__(256) void gptq_qweight_kernel(const uint32_t* __restrict__ packed,
-                                                           uint32_t* __restrict__ qweight, uint32_t N, uint32_t K8) {
-  __shared__ uint32_t tile[64][65];
-  const uint32_t n0 = blockIdx.y * 64, k0 = blockIdx.x * 64;
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
+// GPTQ container -> W4A16 layouts in one launch, both parts transposes bound by HBM.
+//
+// Workgroups from `p_wgs` on: packed [N][K/2] bytes viewed as u32 [N][K/8] -> qweight u32 [K/8][N]:
+// the little-endian word of GPTQ bytes 4kk..4kk+3 of row n holds elements 8kk..8kk+7 of that row at
+// bits 4e (element 2i = low nibble of byte i), which is word (kk, n) of the W4A16 layout.  Each
+// thread transposes a 4 x 4 block of words in registers; a wave's 8 x 8 threads make both its loads
+// and its stores whole 128-byte lines (16 bytes a lane, at any 4-byte alignment), with no LDS.
+// The first `p_wgs` (their loads and barrier then overlap the rest's streams; last, they were a tail
+// of 1.3 us): 64 columns x 32 groups of the parameters through LDS.  scales f32 [N][G] -> bf16 [G][N]
+// (RNE); zeros i32 [N][G] -> u32 [G][N/8] (nibble e of word j = zero of column 8j + e).
+// 11008 x 4096, group 128 (48.8 MB read and written): 17.0 us as two launches of 4-byte
+// transposes (the parameters read at a stride of one row per lane), 9.7 us now, 5.0 TB/s; 14336 x
+// 14336 (221 MB) 46.8 us, 4.8 TB/s, where a copy of that size reaches 5.2.  Two or four blocks per
+// thread measured the same or slower.
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int kGptqTileN = 64, kGptqTileG = 32;
+__global__ __launch_bounds__(256) void gptq_convert_kernel(const uint32_t* __restrict__ packed,
+                                                           const float* __restrict__ s,
+                                                           const int32_t* __restrict__ z,
+                                                           uint32_t* __restrict__ qweight,
+                                                           uint16_t* __restrict__ s_out,
+                                                           uint32_t* __restrict__ z_out, uint32_t N, uint32_t K8,
+                                                           uint32_t G, uint32_t p_wgs) {
+  __shared__ float st[kGptqTileG][kGptqTileN + 1];
+  __shared__ uint32_t zt[kGptqTileG][kGptqTileN + 1];
+  const uint32_t t = threadIdx.x;
+  if (blockIdx.x >= p_wgs) {
+    const uint32_t kt = (K8 + 63) / 64, wave = t >> 6, lane = t & 63, b = blockIdx.x - p_wgs;
+    const uint32_t k0 = (b % kt) * 64 + (wave & 1) * 32 + (lane & 7) * 4;
+    const uint32_t n0 = (b / kt) * 64 + (wave >> 1) * 32 + (lane >> 3) * 4;
+    if (n0 >= N || k0 >= K8) return;  // N % 8 == 0: the four columns are in range together
+    u32x4 v[4];
+    if (k0 + 4 <= K8) {
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint32_t n = n0 + ty + 4 * i, kk = k0 + tx;
-    if (n < N && kk < K8) tile[ty + 4 * i][tx] = packed[(size_t)n * K8 + kk];
+      for (int i = 0; i < 4; ++i) v[i] = *(const u32x4_a4*)(packed + (size_t)(n0 + i) * K8 + k0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[i][j] = k0 + j < K8 ? packed[(size_t)(n0 + i) * K8 + k0 + j] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (k0 + j < K8)
+        *(u32x4_a4*)(qweight + (size_t)(k0 + j) * N + n0) = u32x4{v[0][j], v[1][j], v[2][j], v[3][j]};
+    return;
+  }
+  const uint32_t gt = (G + kGptqTileG - 1) / kGptqTileG, b = blockIdx.x;
+  const uint32_t g0 = (b % gt) * kGptqTileG, n0 = (b / gt) * kGptqTileN;
+#pragma unroll
+  for (int i = 0; i < kGptqTileN * kGptqTileG / 256; ++i) {
+    const uint32_t e = t + 256 * i, n = n0 + e / kGptqTileG, g = g0 + e % kGptqTileG;
+    if (n < N && g < G) {
+      st[e % kGptqTileG][e / kGptqTileG] = s[(size_t)n * G + g];
+      zt[e % kGptqTileG][e / kGptqTileG] = (uint32_t)z[(size_t)n * G + g];
+    }
   }
   __syncthreads();
+  const uint32_t g = g0 + t / 8, c = (t % 8) * 8, n = n0 + c;  // 8 columns of one group
+  if (g >= G || n >= N) return;
+  const float* sr = &st[t / 8][c];
+  const uint32_t* zr = &zt[t / 8][c];
+  uint16_t* so = s_out + (size_t)g * N + n;
+  uint32_t zw = 0;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint32_t kk = k0 + ty + 4 * i, n = n0 + tx;
-    if (n < N && kk < K8) qweight[(size_t)kk * N + n] = tile[tx][ty + 4 * i];
-  }
-}
-
-// scales f32 [N][G] -> bf16 [G][N] (RNE); zeros i32 [N][G] -> u32 [G][N/8]
-// (nibble e of word j = zero of column 8j + e).  One thread per output word
-// of zeros, i.e. 8 columns of one group.
-__global__ __launch_bounds__(256) void gptq_params_kernel(const float* __restrict__ s, const int32_t* __restrict__ z,
-                                                          uint16_t* __restrict__ s_out, uint32_t* __restrict__ z_out,
-                                                          uint32_t N, uint32_t G) {
-  const uint32_t words = N / 8;
-  const size_t total = (size_t)G * words;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-    const uint32_t g = (uint32_t)(i / words), j = (uint32_t)(i % words);
-    uint32_t zw = 0;
+  for (int e = 0; e < 8; ++e) zw |= (zr[e] & 0xFu) << (4 * e);
+  if (((uintptr_t)s_out & 15) == 0) {
+    *(u32x4*)so = u32x4{pack_bf16x2(sr[0], sr[1]), pack_bf16x2(sr[2], sr[3]), pack_bf16x2(sr[4], sr[5]),
+                        pack_bf16x2(sr[6], sr[7])};
+  } else {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint32_t n = 8 * j + e;
-      s_out[(size_t)g * N + n] = f32_to_bf16_rne(s[(size_t)n * G + g]);
-      zw |= ((uint32_t)z[(size_t)n * G + g] & 0xFu) << (4 * e);
-    }
-    z_out[i] = zw;
+    for (int e = 0; e < 8; ++e) so[e] = f32_to_bf16_rne(sr[e]);
   }
+  z_out[(size_t)g * (N / 8) + n / 8] = zw;
 }
 
 }  // namespace t0mi
@@ -314,13 +347,12 @@ extern "C" int t0mi_gptq_convert(t0mi_ctx* ctx, uint64_t packed, uint64_t scales
     return set_error(T0MI_ERR_INVALID, "misaligned buffer (4-byte sections, 2-byte bf16 scales)");
   if (rows == 0 || cols == 0 || ctx->null_backend) return T0MI_OK;
   const uint32_t K8 = cols / 8, G = cols / group;
-  hipLaunchKernelGGL(gptq_qweight_kernel, dim3((K8 + 63) / 64, (rows + 63) / 64), dim3(256), 0, ctx->stream,
-                     (const uint32_t*)packed, (uint32_t*)qweight, rows, K8);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return hip_fail(e, "gptq qweight launch");
-  hipLaunchKernelGGL(gptq_params_kernel, dim3(grid_for(ctx, (size_t)G * (rows / 8))), dim3(256), 0, ctx->stream,
-                     (const float*)scales_f32, (const int32_t*)zeros_i32, (uint16_t*)scales_bf16, (uint32_t*)qzeros,
-                     rows, G);
-  e = hipGetLastError();
-  return e == hipSuccess ? T0MI_OK : hip_fail(e, "gptq params launch");
+  const uint64_t q_wgs = (uint64_t)((K8 + 63) / 64) * ((rows + 63) / 64);
+  const uint64_t p_wgs =
+      (uint64_t)((G + kGptqTileG - 1) / kGptqTileG) * ((rows + kGptqTileN - 1) / kGptqTileN);
+  hipLaunchKernelGGL(gptq_convert_kernel, dim3((uint32_t)(q_wgs + p_wgs)), dim3(256), 0, ctx->stream,
+                     (const uint32_t*)packed, (const float*)scales_f32, (const int32_t*)zeros_i32, (uint32_t*)qweight,
+                     (uint16_t*)scales_bf16, (uint32_t*)qzeros, rows, K8, G, (uint32_t)p_wgs);
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess ? T0MI_OK : hip_fail(e, "gptq conversion launch");
 }
