@@ -109,6 +109,8 @@ struct t0mi_ctx {
 namespace t0mi {
 // Grows ctx->ws to at least `bytes` (waits for the stream first).
 int ensure_workspace(t0mi_ctx* ctx, size_t bytes);
+// Whether ctx->ws holds `bytes` or may grow to (no capture, no live graph holding its address).
+bool workspace_available(t0mi_ctx* ctx, size_t bytes);
 // Grows ctx->cvt to at least `bytes` (waits for the stream first).
 int ensure_cvt_buffer(t0mi_ctx* ctx, size_t bytes);
 // Counters of the XCD exchange, per XCD: at most this many tiles per XCD per launch.

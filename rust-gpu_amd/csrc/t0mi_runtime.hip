@@ -124,6 +124,11 @@ int ensure_workspace(t0mi_ctx* ctx, size_t bytes) {
   return T0MI_OK;
 }
 
+bool workspace_available(t0mi_ctx* ctx, size_t bytes) {
+  return bytes <= ctx->ws_bytes ||
+         (ctx->live_graphs.load() == 0 && refuse_if_capturing(ctx, "growing the library workspace") == T0MI_OK);
+}
+
 int ensure_cvt_buffer(t0mi_ctx* ctx, size_t bytes) {
   if (ctx->cvt_bytes >= bytes) return T0MI_OK;
   if (ctx->null_backend) {
@@ -1177,7 +1182,7 @@ static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm
       cached_auto_plan(m, n, k, cfg.transpose, cfg.out_dtype, (uint32_t)ctx->cu_count, &pl)) {
     const uint32_t sk_h = split_k_of(pl.head), sk_t = pl.n1 < n ? split_k_of(pl.tail) : 1;
     const size_t need = std::max(sk_h > 1 ? (size_t)m * pl.n1 * 4 * sk_h : 0, sk_t > 1 ? (size_t)m * (n - pl.n1) * 4 * sk_t : 0);
-    if (need <= ctx->ws_bytes || (ctx->live_graphs.load() == 0 && refuse_if_capturing(ctx, "growth") == T0MI_OK))
+    if (workspace_available(ctx, need))
       return run_gemm_auto(ctx, cfg.transpose, x, b, y, m, n, k, cfg.out_dtype, bias, &chain);
   }
   return run_gemm(ctx, cfg, e, x, b, y, bias, m, n, k, chain);

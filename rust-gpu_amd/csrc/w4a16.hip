@@ -358,6 +358,26 @@ static constexpr uint32_t kDecodeMaxLaunches = 3;
 // need twice the LDS per slab), four for group 128 (the one group whose four-slab
 // registers fit without spilling), three otherwise.
 static uint32_t decode_max_slabs(uint32_t group) { return group == 256 ? 2 : group == 128 ? 4 : 3; }
+// Row tiles of the decode kernel: slabs per workgroup, with the tiles of a call either in one
+// launch (grid.z) or one launch after another.  A workgroup takes about 4.9 + 2.5 us per slab (K =
+// 4096: its activations, at 50 GB/s per CU) and a CU runs one at a time, so one launch costs its
+// rounds of workgroups and pays where the strips leave CUs idle: N = 4096 (64 strips), 100 rows, 27.3
+// -> 10.5 us with four tiles of 2 slabs; 191 rows 44.8 -> 14.1 us with four of 3; 17 rows 9.2 -> 7.4
+// us with two of 1; N = 1376, 191 rows 45.4 -> 11.7 us.  At N = 11008 (172 strips) the tiles of one
+// launch run in two or three rounds (28.9 us at 100 rows) where a launch of 4 slabs and one of 3
+// follow each other on idle CUs (28.4).  Returns the slabs per workgroup of one launch, or 0 for
+// one launch after another.
+static uint32_t decode_row_tiles(uint32_t slabs, uint32_t max_slabs, uint32_t wgs_per_tile, uint32_t cus) {
+  auto rounds = [&](uint32_t wgs) { return (float)((wgs + cus - 1) / cus); };
+  const uint32_t launches = (slabs + max_slabs - 1) / max_slabs;
+  float best = rounds(wgs_per_tile) * (4.9f * launches + 2.5f * slabs) * 0.95f;
+  uint32_t pick = 0;
+  for (uint32_t rs = 1; rs <= max_slabs; ++rs) {
+    const float t = rounds(wgs_per_tile * ((slabs + rs - 1) / rs)) * (4.9f + 2.5f * rs);
+    if (t < best) best = t, pick = rs;
+  }
+  return pick;
+}
 static constexpr uint32_t kPingPongRows = 192;
 static constexpr uint32_t kTwoPassRows = 1536;
 static constexpr uint32_t kSplitRouteRows = 1024;
@@ -674,10 +694,14 @@ extern "C" int t0mi_w4a16_gemm(t0mi_ctx* ctx, uint64_t a, uint64_t qweight, uint
   // launch (one pass over the weights feeds them all), spread evenly over the
   // fewest launches (5 slabs as 3 + 2, not 4 + 1); the other kernels one.
   const uint32_t slabs = (m + 15) / 16;
-  const uint32_t launches = v2 ? (slabs + decode_max_slabs(group) - 1) / decode_max_slabs(group) : slabs;
-  for (uint32_t r0 = 0, done = 0, l = 0, rs = 1; r0 < m; r0 += 16 * rs, done += rs, ++l) {
-    rs = (slabs - done + (launches - l) - 1) / (launches - l);
-    const uint32_t mr = std::min(16u * rs, m - r0);
+  // Planes of every row (several tiles in one launch) only where the workspace may hold them now.
+  uint32_t tile_rs = v2 ? decode_row_tiles(slabs, decode_max_slabs(group), strips * ky, (uint32_t)ctx->cu_count) : 0;
+  if (tile_rs && ky > 1 && !workspace_available(ctx, (size_t)m * n * 4 * ky)) tile_rs = 0;
+  const uint32_t tiles = tile_rs ? (slabs + tile_rs - 1) / tile_rs : 1;
+  const uint32_t launches = tile_rs ? 1 : v2 ? (slabs + decode_max_slabs(group) - 1) / decode_max_slabs(group) : slabs;
+  for (uint32_t r0 = 0, done = 0, l = 0, rs = 1; r0 < m; r0 += 16 * rs * tiles, done += rs, ++l) {
+    rs = tile_rs ? tile_rs : (slabs - done + (launches - l) - 1) / (launches - l);
+    const uint32_t mr = std::min(16u * rs * tiles, m - r0);
     p.a = (const uint16_t*)a + (size_t)r0 * k;
     p.M = mr;
     const size_t ob = out_dtype == T0MI_OUT_BF16 ? 2 : 4;
@@ -692,7 +716,7 @@ extern "C" int t0mi_w4a16_gemm(t0mi_ctx* ctx, uint64_t a, uint64_t qweight, uint
     }
     const bool z = qzeros != 0;
     if (v2) {
-      const dim3 grid(strips, ky), block(nw2 * 64);
+      const dim3 grid(strips, ky, tiles), block(nw2 * 64);
 #define T0MI_W4_V2_RS(NW, G, RS)                                                                               \
   if (z)                                                                                                       \
     hipLaunchKernelGGL((w4a16_decode_v2<NW, KBW2, G / 32, true, G <= 128 ? 4 : 2, RS>), grid, block, 0,        \

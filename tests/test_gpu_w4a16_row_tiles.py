@@ -1,0 +1,59 @@
+"""GPU parity of the W4A16 decode kernel's row tiles in one launch (csrc/w4a16.hip, decode_row_tiles): a
+narrow weight's 64-column strips leave CUs idle, so the slabs of a call run as several tiles of 1 to 4
+slabs side by side.  Every row goes through the operations of a 16-row slab whatever the tile, so the
+f32 results equal, bit for bit, those of the same rows inside a call that tiles them differently; and
+they are within the fp32 bound k * 2^-24 * sum |a w| (times 2) of the exact product.
+Cases: a last tile of one row, of one slab, tiles of 1, 2, 3 and 4 slabs, planes over K (K > 4096) with
+tiles, groups 32 to 256, widths off the strip."""
+import numpy as np
+import pytest
+
+import oracle
+import t0mi
+from gpu_helpers import empty_dev, from_dev, runtime, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def rt():
+    r = runtime()
+    yield r
+    r.close()
+
+
+@pytest.mark.parametrize("m,k,n,group,zeros", [
+    (17, 1024, 520, 128, True),     # two tiles of one slab, the last one row
+    (33, 512, 4096, 64, False),     # three slabs
+    (100, 4096, 1376, 128, True),
+    (129, 512, 1000, 32, True),     # one row past eight slabs
+    (191, 1024, 4096, 128, False),  # four tiles of three slabs
+    (96, 2048, 520, 256, True),     # group 256: at most two slabs a tile
+    (112, 8192, 520, 128, True),    # planes over K and row tiles
+    (150, 512, 6000, 128, False),   # 94 strips
+])
+def test_row_tiles(rt, m, k, n, group, zeros):
+    a = oracle.normal_bf16((m, k), 3 * m + n, 0.0, 1.0)
+    w = oracle.pack_qweight(oracle.nibbles((k, n), m + 1))
+    s = oracle.uniform_bf16((k // group, n), m + 2, 0.005, 0.02)
+    z = oracle.pack_qzeros(oracle.nibbles((k // group, n), m + 3)) if zeros else None
+    da, pa = to_dev(a)
+    dw, pw = to_dev(w)
+    ds, ps = to_dev(s)
+    pz = 0
+    if zeros:
+        dz, pz = to_dev(z)
+
+    def call(r0, rows):
+        dy, py = empty_dev(rows * n * 4, fill=0xCD)
+        rt.w4a16_gemm(pa + r0 * k * 2, pw, ps, pz, 8, py, rows, k, n, group, t0mi.OUT_F32)
+        return from_dev(dy, np.float32, (rows, n))
+
+    y = call(0, m)
+    wf = oracle.dequant_qweight_f32(w, s, z, group, 8).astype(np.float64)
+    af = oracle.bf16_to_f32(a).astype(np.float64)
+    lim = 2 * k * 2.0**-24 * (np.abs(af) @ np.abs(wf))
+    assert (np.abs(y - af @ wf) <= lim).all()
+    for r0, rows in ((0, min(m, 48)), (16, m - 16)):  # other tilings of the same rows, over 16 rows each
+        if rows > 16:
+            assert np.array_equal(call(r0, rows), y[r0:r0 + rows]), (r0, rows)
