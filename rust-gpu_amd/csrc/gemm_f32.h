@@ -23,6 +23,8 @@
 //   * Where the tiles are fewer than the CUs, K is also cut over `pieces` workgroups per tile in
 //     the same launch; their sums are exchanged through memory (xcd_exchange.h) and added in piece
 //     order by the workgroup that arrives last.
+//   * The right operand may also be bf16 and K-contiguous: the inference layer on its cached weight
+//     (bf16_matmul.rs:99-134).
 //   * A tile that would end past the matrix starts earlier instead (it overlaps its neighbour,
 //     whose rows and columns it does not store), so no load needs a column mask.
 //
@@ -34,9 +36,11 @@
 // per tile row and column), and the conversion passes win: f32_plan (gemm_f32_plan.h) draws the line.
 // Measured, forward + data + weight of one layer, before (conversion passes, GEMM, reduce, unpad) and
 // now: 512 tokens, 1024 -> 4096: 66.8 -> 49.8 us; 333 tokens, 1100 -> 770: 56.1 -> 29.8 us; forward
-// alone, 16 x 4096 x 4096: 27.9 -> 17.4 us.  The error against 64-bit sums is the smaller one
+// alone, 16 x 4096 x 4096: 27.9 -> 17.4 us; inference layer, 7 x 11008 x 2048: 12.7 -> 10.6 us.  The error against 64-bit sums is the smaller one
 // (1.9e-7 -> 1.3e-7 relative on the first): K is summed in chains of at most 1024.
 #pragma once
+#include <type_traits>
+
 #include "gemm_bf16_kernel.h"
 #include "gemm_f32_plan.h"
 #include "xcd_exchange.h"
@@ -45,7 +49,7 @@ namespace t0mi {
 
 struct GemmF32Params {
   const float* a;  // K-contiguous: [M][lda]; K-major: [K][lda], M columns
-  const float* b;  // K-contiguous: [N][ldb]; K-major: [K][ldb], N columns
+  const void* b;   // K-contiguous: [N][ldb]; K-major: [K][ldb], N columns; f32 or bf16
   float* y;        // [M][N]
   uint32_t M, N, K, lda, ldb;
   uint32_t a_bytes, b_bytes;  // extent of each operand (below 2 GiB)
@@ -73,7 +77,7 @@ struct F32Tile {
   uint32_t kstep;      // bytes per unit of K
 
   // `first`: the tile's first row (column) of the product; `rows`: the matrix's.
-  __device__ __forceinline__ void init(const float* base, uint32_t bytes, uint32_t ld, int first, int rows, int t) {
+  __device__ __forceinline__ void init(const void* base, uint32_t bytes, uint32_t ld, int first, int rows, int t) {
     rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)bytes, 0x00020000);
     sr = t / PPR;
     sp = t % PPR;
@@ -91,14 +95,13 @@ struct F32Tile {
   // A K tile that K cuts, or that starts past it: zeros there.  A K-contiguous piece that K cuts
   // (K % 4 != 0) is loaded element by element.
   __device__ __forceinline__ void load_cut(int k0, int K, f32x4* v) const {
-    constexpr uint32_t OOB = 0x80000000u;  // past every operand's extent
     const uint32_t ko = (uint32_t)k0 * kstep;
     if (!KM && (K & 3)) {
 #pragma unroll
       for (int i = 0; i < NP; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-          const uint32_t o = k0 + sp * 4 + j < K ? off[i] + ko + (uint32_t)j * 4u : OOB;
+          const uint32_t o = k0 + sp * 4 + j < K ? off[i] + ko + (uint32_t)j * 4u : kF32Oob;
           v[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, (int)o, 0, 0));
         }
     } else {
@@ -106,7 +109,7 @@ struct F32Tile {
       for (int i = 0; i < NP; ++i) {
         const int k = KM ? k0 + sr + i * RSTEP : k0 + sp * 4;
         v[i] = __builtin_bit_cast(
-            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(k < K ? off[i] + ko : OOB), 0, 0));
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(k < K ? off[i] + ko : kF32Oob), 0, 0));
       }
     }
   }
@@ -153,15 +156,58 @@ struct F32Tile {
   }
 };
 
-// BM x BN of Y per workgroup of G groups of WM x WN waves.  AK / BKM: the operand is K-major.
-template <int BM, int BN, int BK, int WM, int WN, int G, int D, bool AK, bool BKM>
+// The same for a bf16 operand, K-contiguous (the cached weight of the inference layer, used in
+// place): pieces of 8 elements go to LDS as they are.  K is a multiple of 8.
+template <int ROWS_, int BK_, int NT>
+struct Bf16Tile {
+  static constexpr int ROWS = ROWS_, BK = BK_;
+  static constexpr int PPR = BK / 8, NP = ROWS * BK / 8 / NT, RSTEP = NT / PPR, KC = BK / 8;
+  static constexpr int ELEMS = ROWS * BK;
+  static_assert(NP * NT * 8 == ROWS * BK && NT % PPR == 0, "whole pieces per thread");
+
+  __amdgpu_buffer_rsrc_t rs;
+  int sr, sp;
+  uint32_t off[NP];
+
+  __device__ __forceinline__ void init(const void* base, uint32_t bytes, uint32_t ld, int first, int rows, int t) {
+    rs = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (int)bytes, 0x00020000);
+    sr = t / PPR;
+    sp = t % PPR;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) off[i] = f32_piece_off(false, ld / 2, first, rows, sr + i * RSTEP, sp);
+  }
+  __device__ __forceinline__ void load_full(int k0, f32x4* v) const {
+    const int so = __builtin_amdgcn_readfirstlane(k0 * 2);
+#pragma unroll
+    for (int i = 0; i < NP; ++i)
+      v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off[i], so, 0));
+  }
+  __device__ __forceinline__ void load_cut(int k0, int K, f32x4* v) const {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const uint32_t o = k0 + sp * 8 < K ? off[i] + (uint32_t)k0 * 2u : kF32Oob;
+      v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)o, 0, 0));
+    }
+  }
+  __device__ __forceinline__ void store_lds(uint16_t* lds, const f32x4* v) const {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) *(f32x4*)(lds + kc_slot<KC>(sr + i * RSTEP, sp) * 8) = v[i];
+  }
+  __device__ __forceinline__ static bf16x8 frag(const uint16_t* lds, int r0, int ks, int lane) {
+    return *(const bf16x8*)(lds + kc_slot<KC>(r0 + (lane & 31), ks * 2 + (lane >> 5)) * 8);
+  }
+};
+
+// BM x BN of Y per workgroup of G groups of WM x WN waves.  AK / BKM: the operand is K-major;
+// B16: the right operand is bf16.
+template <int BM, int BN, int BK, int WM, int WN, int G, int D, bool AK, bool BKM, bool B16 = false>
 __global__ __launch_bounds__(WM* WN* G * 64) void gemm_f32_kernel(GemmF32Params p) {
   constexpr int GT = WM * WN * 64;  // threads per group
   constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32, KS = BK / 16;
   constexpr bool FOLD = gemm_f32_folds(BM, BN);
   constexpr int kFoldTiles = 512 / BK;
   using TA = F32Tile<BM, BK, GT, AK>;
-  using TB = F32Tile<BN, BK, GT, BKM>;
+  using TB = std::conditional_t<B16, Bf16Tile<BN, BK, GT>, F32Tile<BN, BK, GT, BKM>>;
   constexpr int STAGE = TA::ELEMS + TB::ELEMS;  // bf16 elements of one LDS stage
   constexpr int LDO = BN + 4;                   // f32 row length of the output block in LDS
   constexpr int RING_BYTES = G * 2 * STAGE * 2, OUT_BYTES = G * BM * LDO * 4;

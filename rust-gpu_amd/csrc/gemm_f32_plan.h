@@ -49,6 +49,16 @@ constexpr F32Tiles kF32Tiles[] = {
 };
 constexpr int kF32TileCount = sizeof kF32Tiles / sizeof kF32Tiles[0];
 
+// The same for a bf16 right operand (Y = X . WT^T, the inference layer on its cached weight), fitted
+// to 120 random calls of 1 to 64 rows (n 256..14336, k 256..8192); on 120 others the tile picked is 1 %
+// behind the fastest of eight.
+constexpr F32Tiles kWtTiles[] = {
+    {32, 64, 4, {3.827f, 0.268f, 0.311f, 0.646f, 1.522f, 0.378f, 5.687f, 0.451f}},
+    {64, 64, 2, {4.112f, 0.216f, 0.112f, 1.584f, 1.886f, 0.221f, 0.000f, 0.521f}},
+};
+constexpr int kWtTileCount = sizeof kWtTiles / sizeof kWtTiles[0];
+constexpr uint32_t kWtMaxRows = 64;
+
 // First row (column) of the tile that starts at `start`, of `size`, in a matrix of `extent`: a tile
 // that would end past the matrix starts earlier.
 T0MI_HD constexpr int f32_tile_first(int start, int extent, int size) {
@@ -56,11 +66,12 @@ T0MI_HD constexpr int f32_tile_first(int start, int extent, int size) {
   return start < last ? start : last > 0 ? last : 0;
 }
 // Byte offset at K = 0 of 16-byte piece `sp` of source row r of the tile starting at `first`: K-major
-// source rows are K (and the piece 4 columns of the product), others the tile's own rows, clamped.
+// source rows are K (and the piece 4 columns of the product), others the tile's own rows.  Rows past
+// the matrix are past every operand's extent: the range check answers them with zeros and no fetch.
+constexpr uint32_t kF32Oob = 0x80000000u;
 T0MI_HD constexpr uint32_t f32_piece_off(bool kmajor, uint32_t ld, int first, int rows, int r, int sp) {
   if (kmajor) return ((uint32_t)r * ld + (uint32_t)(first + sp * 4)) * 4u;
-  const int row = first + r < rows - 1 ? first + r : rows - 1;
-  return ((uint32_t)row * ld + (uint32_t)(sp * 4)) * 4u;
+  return first + r < rows ? ((uint32_t)(first + r) * ld + (uint32_t)(sp * 4)) * 4u : kF32Oob;
 }
 // First K tile of piece q of p over nkt K tiles (piece q ends where q + 1 starts).
 T0MI_HD constexpr int f32_piece_begin(int q, int p, int nkt) { return (int)((int64_t)q * nkt / p); }
@@ -79,18 +90,19 @@ inline float f32_two_pass_us(uint32_t m, uint32_t n, uint32_t k) {
   return t;
 }
 
-// Y[m,n] over K = k; `split`: the in-launch exchange is available.  A K-major operand narrower
+// The fastest tile of `tab` (and K pieces; `split`: the in-launch exchange is available) for Y[m,n] over
+// K = k, right operand elements of `b_size` bytes, and its time in *us.  A K-major operand narrower
 // than the tile needs a multiple of 4 columns (a 16-byte load may then not straddle the matrix's
 // end); other operands take any size.
-inline F32Plan f32_plan(int mode, uint32_t m, uint32_t n, uint32_t k, uint32_t cus, bool split) {
+inline F32Plan f32_best_tile(const F32Tiles* tab, int count, int mode, int b_size, uint32_t m, uint32_t n, uint32_t k,
+                             uint32_t cus, bool split, float* best_us) {
   F32Plan best;
   if (!m || !n || !k) return best;
-  if ((uint64_t)m * k * 4 >= kF32MaxBytes || (uint64_t)k * n * 4 >= kF32MaxBytes) return best;
+  if ((uint64_t)m * k * 4 >= kF32MaxBytes || (uint64_t)k * n * b_size >= kF32MaxBytes) return best;
   if ((uint64_t)m * n * 4 >= 64 * kF32MaxBytes) return best;
-  float best_us = 0;
   const uint32_t nkt = (k + kF32Bk - 1) / kF32Bk;
-  for (int i = 0; i < kF32TileCount; ++i) {
-    const F32Tiles& t = kF32Tiles[i];
+  for (int i = 0; i < count; ++i) {
+    const F32Tiles& t = tab[i];
     if (f32_a_kmajor(mode) && (int64_t)m < t.bm && m % 4) continue;
     if (f32_b_kmajor(mode) && (int64_t)n < t.bn && n % 4) continue;
     const uint64_t tm = (m + t.bm - 1) / t.bm, tn = (n + t.bn - 1) / t.bn, tiles = tm * tn;
@@ -107,22 +119,48 @@ inline F32Plan f32_plan(int mode, uint32_t m, uint32_t n, uint32_t k, uint32_t c
       float it = (float)((kt + t.groups - 1) / t.groups);
       if (k % 32)  // K-contiguous rows that start inside a 128-byte line
         it *= 1 + 0.5f * ((f32_a_kmajor(mode) ? 0 : t.bm) + (f32_b_kmajor(mode) ? 0 : t.bn)) / (t.bm + t.bn);
-      float us = t.c[0] + t.c[1] * it + (t.c[2] * it + t.c[3]) * (w - 1) +
-                 t.c[6] * ((float)m * n) * 4e-6f / 8 + t.c[7] * ((float)m * k + (float)k * n) * 4e-6f / 8;
+      float us = t.c[0] + t.c[1] * it + (t.c[2] * it + t.c[3]) * (w - 1) + t.c[6] * ((float)m * n) * 4e-6f / 8 +
+                 t.c[7] * ((float)m * k * 4 + (float)k * n * b_size) * 1e-6f / 8;
       if (p > 1) us += t.c[4] + t.c[5] * (float)wgs / 256 * (t.bm * t.bn) / 1024;
-      if (best.tile < 0 || us < best_us) {
+      if (best.tile < 0 || us < *best_us) {
         best.tile = i;
         best.pieces = p;
         best.tiles_m = (uint32_t)tm;
         best.tiles_n = (uint32_t)tn;
-        best_us = us;
+        *best_us = us;
       }
     }
   }
-  // The estimate is 10 % off at small sizes and optimistic at large ones, where the two routes meet
-  // (about 30 GFLOP): there the one launch has to be that much ahead.
-  if (best.tile >= 0 && best_us + 0.2f * (best_us > 15 ? best_us - 15 : 0) > f32_two_pass_us(m, n, k)) best.tile = -1;
   return best;
+}
+// The estimates are 10 % off at small sizes and optimistic at large ones, where the routes meet (f32
+// weights: about 30 GFLOP): there the one launch has to be that much ahead.
+inline bool f32_one_launch_ahead(float us, float other_us) {
+  return us + 0.2f * (us > 15 ? us - 15 : 0) <= other_us;
+}
+
+// Y[m,n] over K = k with f32 operands: a tile of kF32Tiles, or -1.
+inline F32Plan f32_plan(int mode, uint32_t m, uint32_t n, uint32_t k, uint32_t cus, bool split) {
+  float us = 0;
+  F32Plan p = f32_best_tile(kF32Tiles, kF32TileCount, mode, 4, m, n, k, cus, split, &us);
+  if (p.tile >= 0 && !f32_one_launch_ahead(us, f32_two_pass_us(m, n, k))) p.tile = -1;
+  return p;
+}
+
+// Y[m,n] = X[m,k] . WT[n,k]^T, X f32, WT bf16 (k % 8 == 0): a tile of kWtTiles, or -1 for X's
+// conversion and the bf16 routes.  Their times: up to 16 rows and one round of 16-column units the
+// persistent decode kernel (ahead at 1 x 4096 x 4096 alone of what was measured: 9.8 against 10.7
+// us), else the scheduled GEMM with its split-K reduce.
+inline F32Plan wt_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t cus, bool split) {
+  F32Plan p;
+  if (m > kWtMaxRows || k % 8) return p;
+  float us = 0;
+  p = f32_best_tile(kWtTiles, kWtTileCount, F32_DATA, 2, m, n, k, cus, split, &us);
+  const bool decode = m <= 16 && k % 32 == 0 && (uint64_t)n <= 16ull * cus;
+  const float other = decode ? 6.6f + (float)k * (0.00078f + 0.00005f * (float)(m - 1))
+                             : 7.579f + 1.276f * ((float)k * n) * 2e-6f / 8 + 20.56f * ((float)m * k) * 6e-6f / 8;
+  if (p.tile >= 0 && !f32_one_launch_ahead(us, other)) p.tile = -1;
+  return p;
 }
 
 }  // namespace t0mi

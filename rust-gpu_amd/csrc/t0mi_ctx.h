@@ -205,4 +205,6 @@ int run_gemm_persistent(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLa
 // route (f32_plan, operands that overlap Y, an exchange buffer that may not grow now).
 // Asynchronous.
 int run_gemm_f32(t0mi_ctx* ctx, int mode, uint64_t a, uint64_t b, uint64_t y, uint32_t m, uint32_t n, uint32_t k);
+// The same for Y[m,n] = bf16(X)[m,k] . WT[n,k]^T with WT bf16 (k % 8 == 0; wt_plan).
+int run_gemm_wt(t0mi_ctx* ctx, uint64_t x, uint64_t wt, uint64_t y, uint32_t m, uint32_t n, uint32_t k);
 }  // namespace t0mi

@@ -284,6 +284,7 @@ extern "C" int t0mi_matmul_wt_bf16(t0mi_ctx* ctx, uint64_t x, uint64_t wt_bf16, 
   if (k % 8 || n % 8) return set_error(T0MI_ERR_INVALID, "K=%u and N=%u must be multiples of 8 (WT is used in place)", k, n);
   if (wt_bf16 & 15) return set_error(T0MI_ERR_INVALID, "WT must be 16-byte aligned");
   if (m == 0 || n == 0) return T0MI_OK;
+  if ((rc = run_gemm_wt(ctx, x, wt_bf16, y, m, n, k)) <= 0) return rc;
   rc = ensure_cvt_buffer(ctx, align256((size_t)m * k * 2));
   if (rc) return rc;
   if (ctx->null_backend) return T0MI_OK;

@@ -25,7 +25,12 @@ static void operand(bool km, int size, uint32_t ld, int rows, int K, int first, 
   const bool whole = k0 + kF32Bk <= K;
   for (int r = 0; r < srows; ++r)
     for (int sp = 0; sp < ppr; ++sp) {
-      const uint64_t off = f32_piece_off(km, ld, first, rows, r, sp) + (uint64_t)k0 * (km ? ld * 4u : 4u);
+      const uint32_t at0 = f32_piece_off(km, ld, first, rows, r, sp);
+      if (at0 == kF32Oob) {  // zeros by the range check: only rows past the matrix
+        check(!km && first + r >= rows && bytes < kF32MaxBytes, "row past the matrix", mode, m, n, k);
+        continue;
+      }
+      const uint64_t off = at0 + (uint64_t)k0 * (km ? ld * 4u : 4u);
       if (km) {
         if (!whole && k0 + r >= K) continue;  // zeros by the range check
         // Columns past the matrix are read (and never stored); a piece that leaves the operand must
@@ -42,20 +47,8 @@ static void operand(bool km, int size, uint32_t ld, int rows, int K, int first, 
     }
 }
 
-static void one(int mode, unsigned m, unsigned n, unsigned k, int split, std::vector<int>& used) {
-  const F32Plan p = f32_plan(mode, m, n, k, 256, split);
-  if (p.tile < 0) {
-    ++used[kF32TileCount * 4];
-    return;
-  }
-  const F32Tiles& t = kF32Tiles[p.tile];
-  int lp = 0;
-  while ((1u << lp) < p.pieces) ++lp;
-  ++used[p.tile * 4 + lp];
-  check(split || p.pieces == 1, "pieces without the exchange", mode, m, n, k);
-  check((uint64_t)p.tiles_m * p.tiles_n * p.pieces * t.bm * t.bn * 4 <= kF32SlotBytes || p.pieces == 1, "slots", mode, m,
-        n, k);
-  // Outputs: each row (and column) is stored by exactly one tile row (column).
+// Outputs: each row (and column) is stored by exactly one tile row (column); K pieces cover K once.
+static void cover(const F32Plan& p, const F32Tiles& t, int mode, unsigned m, unsigned n, unsigned k) {
   for (int d = 0; d < 2; ++d) {
     const int ext = d ? (int)n : (int)m, size = d ? t.bn : t.bm, tiles = d ? (int)p.tiles_n : (int)p.tiles_m;
     std::vector<int> hit(ext, 0);
@@ -68,6 +61,8 @@ static void one(int mode, unsigned m, unsigned n, unsigned k, int split, std::ve
     for (int h : hit) ok = ok && h == 1;
     check(ok, "coverage", mode, m, n, k);
   }
+  check((uint64_t)p.tiles_m * p.tiles_n * p.pieces * t.bm * t.bn * 4 <= kF32SlotBytes || p.pieces == 1, "slots", mode, m,
+        n, k);
   const int nkt = ((int)k + kF32Bk - 1) / kF32Bk;
   check(f32_piece_begin(0, (int)p.pieces, nkt) == 0 && f32_piece_begin((int)p.pieces, (int)p.pieces, nkt) == nkt,
         "K range", mode, m, n, k);
@@ -76,6 +71,41 @@ static void one(int mode, unsigned m, unsigned n, unsigned k, int split, std::ve
     check(b < e, "empty piece", mode, m, n, k);
     check(gemm_f32_folds(t.bm, t.bn) || (uint32_t)(e - b) * kF32Bk <= kF32ChainMax, "chain", mode, m, n, k);
   }
+}
+
+// The bf16 weight's route: n and k multiples of 8 (what the entry point takes), up to 64 rows.
+static void wt(unsigned m, unsigned n, unsigned k, int split, int* used) {
+  const F32Plan p = wt_plan(m, n, k, 256, split);
+  if (p.tile < 0) return;
+  ++used[p.tile];
+  const F32Tiles& t = kWtTiles[p.tile];
+  check(m <= kWtMaxRows && (split || p.pieces == 1), "wt range", 3, m, n, k);
+  cover(p, t, 3, m, n, k);
+  const uint64_t bytes = (uint64_t)n * k * 2;
+  for (int tn : {0, (int)p.tiles_n - 1})
+    for (int kt : {0, ((int)k - 1) / kF32Bk})
+      for (int r = 0; r < t.bn; ++r)
+        for (int sp = 0; sp < kF32Bk / 8; ++sp) {
+          const int first = f32_tile_first(tn * t.bn, (int)n, t.bn);
+          const uint32_t at0 = f32_piece_off(false, k / 2, first, (int)n, r, sp);
+          if (at0 == kF32Oob || kt * kF32Bk + sp * 8 >= (int)k) continue;
+          check((uint64_t)at0 + (uint64_t)kt * kF32Bk * 2 + 16 <= bytes, "wt load", 3, m, n, k);
+        }
+}
+
+static void one(int mode, unsigned m, unsigned n, unsigned k, int split, std::vector<int>& used) {
+  const F32Plan p = f32_plan(mode, m, n, k, 256, split);
+  if (p.tile < 0) {
+    ++used[kF32TileCount * 4];
+    return;
+  }
+  const F32Tiles& t = kF32Tiles[p.tile];
+  int lp = 0;
+  while ((1u << lp) < p.pieces) ++lp;
+  ++used[p.tile * 4 + lp];
+  check(split || p.pieces == 1, "pieces without the exchange", mode, m, n, k);
+  cover(p, t, mode, m, n, k);
+  const int nkt = ((int)k + kF32Bk - 1) / kF32Bk;
   // Loads: first, second last and last tile of each dimension, first and last K tiles.
   for (int kt : {0, nkt / 2, nkt - 1})
     for (int back = 0; back < 2; ++back) {
@@ -102,6 +132,12 @@ int main() {
         one(mode, m, n, k, split, used);
       }
     }
+  int wt_used[kWtTileCount] = {};
+  for (int split = 0; split < 2; ++split)
+    for (int i = 0; i < 4000; ++i)
+      wt(1 + (unsigned)rand() % 70, 8 * (1 + (unsigned)rand() % (1u << (1 + rand() % 11))),
+         8 * (1 + (unsigned)rand() % (1u << (1 + rand() % 10))), split, wt_used);
+  for (int i = 0; i < kWtTileCount; ++i) g_fail += wt_used[i] == 0;
   for (int i = 0; i < kF32TileCount; ++i)
     printf("%dx%d pieces 1/2/4/8: %d %d %d %d\n", kF32Tiles[i].bm, kF32Tiles[i].bn, used[i * 4], used[i * 4 + 1],
            used[i * 4 + 2], used[i * 4 + 3]);

@@ -100,6 +100,39 @@ def test_f32_product(rt, mode, m, n, k):
         assert th.equal(y, z), "a second call differs"
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 8, 8), (3, 200, 40),   # one cut K tile, columns short of the tile
+    (7, 11008, 2048),          # 32x64
+    (17, 520, 3000),           # 32x64, K pieces, K % 32 != 0
+    (16, 512, 8192),           # 8 pieces
+    (33, 1000, 264), (64, 4096, 1032),  # two row tiles / 64x64
+    (64, 72, 4096),
+])
+def test_bf16_weight(rt, m, n, k):
+    """matmul_with_wt_bf16 (bf16_matmul.rs:99-134): X f32, WT bf16 in place; same bars."""
+    th = torch()
+    for ints in (True, False):
+        a, _, exact, mag = operands("forward", m, n, k, ints)
+        g = th.Generator(device="cuda:0").manual_seed(m * 7 + n * 3 + k)
+        th.randn(m, k, generator=g, device="cuda:0")
+        b = th.randn(k, n, generator=g, device="cuda:0")  # operands()' second draw
+        if ints:
+            b = (b * 3).round().clamp(-8, 8)
+        wt = th.full((n * k + 512,), float("nan"), device="cuda:0", dtype=th.bfloat16)
+        w = wt[256:256 + n * k].view(n, k)
+        w.copy_(b.t())
+        buf = th.full((m * n + 1024,), 7.5, device="cuda:0")
+        y = buf[:m * n].view(m, n)
+        y.fill_(float("nan"))
+        rt.matmul_with_wt_bf16(a.data_ptr(), w.data_ptr(), y.data_ptr(), m, k, n)
+        th.cuda.synchronize()
+        assert bool((buf[m * n:] == 7.5).all()), "wrote past Y"
+        if ints:
+            assert th.equal(y.double(), exact)
+        else:
+            assert bool(((y.double() - exact).abs() <= 4 * k**0.5 * 2.0**-24 * mag + 1e-30).all())
+
+
 def test_f32_product_against_oracle(rt):
     m, n, k = 333, 770, 1100
     th = torch()
