@@ -718,7 +718,13 @@ extern "C" int t0mi_w4a16_gemm(t0mi_ctx* ctx, uint64_t a, uint64_t qweight, uint
     if (v2) {
       const dim3 grid(strips, ky, tiles), block(nw2 * 64);
 #define T0MI_W4_V2_RS(NW, G, RS)                                                                               \
-  if (z)                                                                                                       \
+  if (z && tiles > 1)                                                                                          \
+    hipLaunchKernelGGL((w4a16_decode_v2<NW, KBW2, G / 32, true, G <= 128 ? 4 : 2, RS, false, true>), grid,     \
+                       block, 0, ctx->stream, p);                                                              \
+  else if (tiles > 1)                                                                                          \
+    hipLaunchKernelGGL((w4a16_decode_v2<NW, KBW2, G / 32, false, G <= 128 ? 4 : 2, RS, false, true>), grid,    \
+                       block, 0, ctx->stream, p);                                                              \
+  else if (z)                                                                                                  \
     hipLaunchKernelGGL((w4a16_decode_v2<NW, KBW2, G / 32, true, G <= 128 ? 4 : 2, RS>), grid, block, 0,        \
                        ctx->stream, p);                                                                        \
   else                                                                                                         \

@@ -100,7 +100,8 @@ __device__ __forceinline__ float bf16f(uint32_t h) { return __builtin_bit_cast(f
 // RS row slabs of 16 (1..4) share one pass over the weights: each dequantized
 // weight fragment feeds every slab's MFMAs, and every row goes through exactly
 // the operations of a 16-row launch on its own slab (bit-identical results).
-// grid.z workgroups per strip take one tile of RS slabs each.
+// TILES: grid.z workgroups per strip take one tile of RS slabs each (a kernel of
+// its own: the tile's addresses cost the one-tile decode 3 %, 7.9 -> 8.2 us).
 //
 // XK (one slab): a 1-D grid of strips x p.pieces workgroups numbered for the
 // XCD exchange (xcd_exchange.h); piece c of a strip covers k-blocks
@@ -109,11 +110,11 @@ __device__ __forceinline__ float bf16f(uint32_t h) { return __builtin_bit_cast(f
 // device-scope policy (normally all on the strip's XCD) and the last piece sums
 // them in piece order and stores Y, all in this launch: every CU gets several
 // workgroups however few strips N has.
-template <int NW, int KBW, int KBPG, bool ZEROS, int CH = 1, int RS = 1, bool XK = false>
+template <int NW, int KBW, int KBPG, bool ZEROS, int CH = 1, int RS = 1, bool XK = false, bool TILES = false>
 __global__ __launch_bounds__(NW * 64) void w4a16_decode_v2(W4Params p) {
   static_assert(KBW % KBPG == 0, "whole groups per wave");
   static_assert(RS >= 1 && RS <= 4, "one to four row slabs");
-  static_assert(!XK || RS == 1, "the in-launch K split runs one slab");
+  static_assert(!XK || (RS == 1 && !TILES), "the in-launch K split runs one slab");
   // CH chunks per wave: chunk c's loads are issued, then its blocks computed,
   // before chunk c+1's loads (CB blocks, whole groups and pairs per chunk).
   constexpr int CB = KBW / CH;
@@ -128,11 +129,12 @@ __global__ __launch_bounds__(NW * 64) void w4a16_decode_v2(W4Params p) {
     if (strip >= p.strips) return;  // the numbering's padding (whole workgroup)
     xk_check_placement(p.xk);
   }
-  // grid.z: row tiles of RS slabs (the last one may hold fewer rows).
-  const uint32_t row0 = XK ? 0u : blockIdx.z * (16 * RS);
-  p.a += (size_t)row0 * p.K;
-  p.y = (char*)p.y + (size_t)row0 * p.N * (p.out_bf16 && gridDim.y == 1 ? 2 : 4);
-  p.M = p.M - row0;
+  if constexpr (TILES) {  // grid.z: row tiles of RS slabs (the last one may hold fewer rows)
+    const uint32_t row0 = blockIdx.z * (16 * RS);
+    p.a += (size_t)row0 * p.K;
+    p.y = (char*)p.y + (size_t)row0 * p.N * (p.out_bf16 && gridDim.y == 1 ? 2 : 4);
+    p.M -= row0;
+  }
   const int n0 = (int)strip * 64;
   const int ncol = n0 + 4 * c;
   const bool col_ok = ncol < (int)p.N;  // N % 8 == 0, so the whole quad is in range
