@@ -320,16 +320,15 @@ __global__ __launch_bounds__(WM* WN* G * 64) void gemm_f32_kernel(GemmF32Params 
   };
   const int nfull = (K / BK - kb) / G;  // tiles i < nfull are whole in every group
   int i = 0;
-  for (; i + 2 * D < nfull; i += D) {
-    if (FOLD && i % kFoldTiles == 0) fold();
-    static_for<D>([&](auto sc) { iteration(i + decltype(sc)::value, sc, Whole{}); });
+  while (i + 2 * D < nfull) {
+    const int stop = FOLD ? min(nfull - 2 * D, i + kFoldTiles) : nfull - 2 * D;
+    for (; i < stop; i += D) static_for<D>([&](auto sc) { iteration(i + decltype(sc)::value, sc, Whole{}); });
+    if (FOLD) fold();
   }
-  for (; i < nit; i += D) {
-    if (FOLD && i % kFoldTiles == 0) fold();
+  for (; i < nit; i += D)
     static_for<D>([&](auto sc) {
       if (i + decltype(sc)::value < nit) iteration(i + decltype(sc)::value, sc, Cut{});
     });
-  }
   if (FOLD) fold();
 
   // Lane l of block (fn, fm) holds row fm*32 + (l & 31), columns fn*32 + 8*g + 4*(l >> 5) + 0..3.
