@@ -29,7 +29,8 @@
 //        4e + l/4, e = 0..3.
 // Output: f32 or bf16 (round to nearest even), after an optional fused epilogue chain.
 // Split-K: partition p covers K range [p*Kp, (p+1)*Kp) and writes its own f32
-// plane at Y + p*y_split_stride (src/t0/gemm_gen.rs:760-793).
+// plane at Y + p*y_split_stride (src/t0/gemm_gen.rs:760-793); gemm_bf16_exchange_kernel sums two
+// partitions in the launch instead.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -38,6 +39,7 @@
 
 #include "epi_chain.h"
 #include "index_maps.h"
+#include "xcd_exchange.h"
 
 namespace t0mi {
 
@@ -446,10 +448,52 @@ struct GemmTile {
   static_assert(!EVEN || LPT * (S - 1) <= 63, "vmcnt range");
 };
 
+// Sums a tile's two K partitions in partition order, in the launch that computed them: each workgroup
+// stores its accumulators in its slot, and the one that arrives last at the tile (true returned) has the
+// sum in acc, the same to the bit as t0mi_splitk_reduce's.  Slots are in fragment order (store i of a
+// workgroup writes 16 bytes a thread); rows past M (`row`: the lane's first) are neither written nor read.
+template <int FM, int FN, int NTHR>
+__device__ __forceinline__ bool exchange_partitions(f32x16 (&acc)[FN][FM], const XcdExchange& x, uint32_t tile,
+                                                    uint32_t part, int row, int M) {
+  constexpr uint32_t SLOT = FM * FN * NTHR * 64;  // bytes
+  const __amdgpu_buffer_rsrc_t slots = xk_slots(x.part + (size_t)tile * (SLOT / 2), 2 * SLOT);
+  const uint32_t off = threadIdx.x * 16;
+  auto at = [&](int fm, int fn, int g) { return off + (uint32_t)(((fm * FN + fn) * 4 + g) * (NTHR * 16)); };
+  static_for<FM>([&](auto fmc) {
+    constexpr int fm = decltype(fmc)::value;
+    if (row + fm * 32 < M)
+      static_for<FN>([&](auto fnc) {
+        constexpr int fn = decltype(fnc)::value;
+        const f32x16& a = acc[fn][fm];
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          xk_store(slots, part * SLOT + at(fm, fn, g), xk_f32x4{a[g * 4], a[g * 4 + 1], a[g * 4 + 2], a[g * 4 + 3]});
+      });
+  });
+  if (!xk_arrive(x, tile, 2)) return false;
+  static_for<FM>([&](auto fmc) {
+    constexpr int fm = decltype(fmc)::value;
+    if (row + fm * 32 < M)
+      static_for<FN>([&](auto fnc) {
+        constexpr int fn = decltype(fnc)::value;
+        xk_f32x4 t[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) t[g] = xk_load(slots, (part ^ 1) * SLOT + at(fm, fn, g));
+        // the sum of two does not depend on their order
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[fn][fm][r] += t[r / 4][r % 4];
+      });
+  });
+  xk_reset(x, tile);
+  return true;
+}
+
 // One output tile (tm, tn) of K partition `part`: the whole kernel body, called
-// once by gemm_bf16_kernel and in a loop by the persistent kernel.
-template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
-__device__ __forceinline__ void gemm_bf16_tile(const GemmParams& p, int tm, int tn, int part) {
+// once by gemm_bf16_kernel and in a loop by the persistent kernel.  XK: the two partitions of a
+// tile are summed through `xk` (p.y, p.ldy: the final output); otherwise each partition stores its plane.
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN, bool XK = false>
+__device__ __forceinline__ void gemm_bf16_tile(const GemmParams& p, int tm, int tn, int part,
+                                               const XcdExchange* xk = nullptr) {
   using T = GemmTile<BM, BN, BK, WM, WN, S, NN>;
   constexpr int FM = T::FM, FN = T::FN, KC = T::KC, KS = T::KS, NC = T::NC;
   constexpr int TM = T::TM, TN = T::TN;
@@ -790,7 +834,12 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmParams& p, int tm, int 
   // i.e. four consecutive columns per (lane, g): one 16-byte (f32) or
   // 8-byte (bf16) store.  The (fm, fn) loops are expanded at compile time so
   // acc is only ever indexed by constants and stays in registers.
-  const bool partial_plane = p.split_k > 1;
+  if constexpr (XK) {
+    if (!exchange_partitions<FM, FN, T::NTHR>(acc, *xk, (uint32_t)tm + (uint32_t)tn * p.tiles_m, (uint32_t)part,
+                                              m0 + wm * TM + (lane & 31), (int)p.M))
+      return;
+  }
+  const bool partial_plane = !XK && p.split_k > 1;
   char* ybase = (char*)p.y + (partial_plane ? (size_t)part * p.y_split_stride : 0);
   // Full tiles with bf16 output: stage each wave's block through the (now
   // idle) LDS ring and store whole rows, when the blocks fit in it.
@@ -810,6 +859,14 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_kernel(GemmParams p) {
   int tm, tn, part;
   tile_coords(p, tm, tn, part);
   gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN>(p, tm, tn, part);
+}
+
+// A kernel of its own, so that launches without the exchange keep their registers.
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_exchange_kernel(GemmParams p, XcdExchange xk) {
+  int tm, tn, part;
+  tile_coords(p, tm, tn, part);
+  gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, true>(p, tm, tn, part, &xk);
 }
 
 }  // namespace t0mi

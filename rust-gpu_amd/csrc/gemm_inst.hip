@@ -26,6 +26,25 @@ static void launch_variant(dim3 g, hipStream_t s, const GemmParams& p) {
   hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, BK, WM, WN, S, NN>), g, dim3(WM * WN * 64), 0, s, p);
 }
 
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
+static void launch_exchange(dim3 g, hipStream_t s, const GemmParams& p, const XcdExchange& x) {
+  hipLaunchKernelGGL((gemm_bf16_exchange_kernel<BM, BN, BK, WM, WN, S, NN>), g, dim3(WM * WN * 64), 0, s, p, x);
+}
+// Split-K summed in the launch: 64x64 tiles in two partitions (run_gemm).  The exchange costs the last
+// workgroup of a tile one slot of 16 KB, the reduce launch it replaces about 1.5-2.5 us.  60 random calls
+// that the ranked schedule gives that split: 1.05 times as fast (0.99 at the least: 4x480x1600), and the
+// call issues one launch less (100x1000x1032: 7.4 -> 6.4 us where the host's enqueue shows).  With more to
+// sum in one workgroup the reduce over the whole chip is faster: 64x64 in 4 partitions 7.6 -> 8.7 us
+// (9x2432x2712), in 8 parts 8.7 -> 10.2 (12x1536x7592); 64x128 in 2 parts 11.0 -> 11.4 (2x10096x1560), in 4
+// parts 9.6 -> 11.0 (8x6088x2448); 128x128 in 2 parts 16.4 -> 17.8 (68x10712x2688).
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
+static constexpr GemmExchangeFn exchange_of() {
+  if constexpr (BM == 64 && BN == 64 && BK == 64 && WM * WN == 4)
+    return launch_exchange<BM, BN, BK, WM, WN, S, NN>;
+  else
+    return nullptr;
+}
+
 #define T0MI_V(BM, BN, BK, WM, WN, S)                                                                  \
   static void launch_##BM##_##BN##_##BK##_##WM##_##WN##_##S(dim3 g, hipStream_t s, const GemmParams& p) { \
     launch_variant<BM, BN, BK, WM, WN, S, (T0MI_INST_NN != 0)>(g, s, p);                              \
@@ -40,7 +59,8 @@ static void launch_variant(dim3 g, hipStream_t s, const GemmParams& p) {
 
 static const GemmLaunchEntry kTable[] = {
 #define T0MI_V(BM, BN, BK, WM, WN, S) \
-  {BM, BN, BK, WM, WN, S, T0MI_INST_NN, launch_##BM##_##BN##_##BK##_##WM##_##WN##_##S},
+  {BM, BN, BK, WM, WN, S, T0MI_INST_NN, launch_##BM##_##BN##_##BK##_##WM##_##WN##_##S, \
+   exchange_of<BM, BN, BK, WM, WN, S, (T0MI_INST_NN != 0)>()},
 #include "gemm_variants.def"
 #undef T0MI_V
 #undef T0MI_V_NT

@@ -19,9 +19,11 @@ struct XcdExchange;  // xcd_exchange.h
 namespace t0mi {
 
 typedef void (*GemmLaunchFn)(dim3 grid, hipStream_t stream, const GemmParams& p);
+typedef void (*GemmExchangeFn)(dim3 grid, hipStream_t stream, const GemmParams& p, const XcdExchange& x);
 struct GemmLaunchEntry {
   int bm, bn, bk, wm, wn, stages, nn;
   GemmLaunchFn fn;
+  GemmExchangeFn fn_exchange;  // split-K summed inside the launch; null where that does not pay
 };
 // Tables defined by the gemm_inst.hip objects (one per variant block and layout).
 const GemmLaunchEntry* gemm_table_p0_nt(size_t* n);
@@ -119,6 +121,8 @@ int ensure_cvt_buffer(t0mi_ctx* ctx, size_t bytes);
 // time (176 tickets on one line: 19 us for a 8 us decode).
 constexpr uint32_t kXkCountersPerXcd = 1024;
 constexpr uint32_t kXkCounterStride = 64;  // u32s between counters
+// Partial slots of a bf16 GEMM that sums its K partitions in the launch, at most.
+constexpr size_t kExchangeSlotBytes = 32u << 20;
 // Readies the XCD exchange for a launch of `tiles` tiles with `part_bytes` of
 // partial slots: false (no error set) when the device's placement did not
 // check out or the tiles do not fit the counters; T0MI_ERR_* when a buffer
@@ -153,7 +157,9 @@ int run_gemm_planned(t0mi_ctx* ctx, const AutoPlan& pl, uint32_t transpose, uint
                      uint32_t m, uint32_t n, uint32_t k, uint32_t out_dtype = T0MI_OUT_F32, uint64_t bias = 0,
                      const EpiChain* epi = nullptr);
 // Launches the bf16 GEMM kernel for (cfg, params) on ctx's stream.
-int launch_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e, GemmParams p);
+// With `x` the K partitions are summed inside the launch (p.y and p.ldy: the final output).
+int launch_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e, GemmParams p,
+                const XcdExchange* x = nullptr);
 int check_ctx(t0mi_ctx* ctx);
 // T0MI_ERR_CAPTURE when ctx's stream is being captured into a graph (calls
 // that wait, allocate or copy to the host cannot be recorded); `what` names

@@ -183,7 +183,8 @@ int xk_prepare(t0mi_ctx* ctx, uint32_t tiles, size_t part_bytes, XcdExchange* x,
   return T0MI_OK;
 }
 
-int launch_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e, GemmParams p) {
+int launch_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e, GemmParams p,
+                const XcdExchange* x) {
   const uint32_t nwg = p.tiles_m * p.tiles_n * p.split_k;
   if (nwg == 0) return T0MI_OK;
   // Grid axes follow the reference convention (swap_grid: x -> N tiles); the
@@ -196,7 +197,10 @@ int launch_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntr
   // with more tiles than CUs, normal stores are faster).
   p.stream_out = nwg <= (uint32_t)ctx->cu_count;
   if (ctx->null_backend) return T0MI_OK;
-  e->fn(grid, ctx->stream, p);
+  if (x)
+    e->fn_exchange(grid, ctx->stream, p, *x);
+  else
+    e->fn(grid, ctx->stream, p);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return hip_fail(err, "gemm launch");
   return T0MI_OK;
@@ -997,9 +1001,19 @@ int run_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* 
     return launch_gemm(ctx, cfg, e, p);
   }
   // Split-K: partitions of whole K tiles write f32 planes into the workspace,
-  // then a reduce pass sums them in partition order.
+  // then a reduce pass sums them in partition order; or, where that is faster (exchange_of in
+  // gemm_inst.hip), the last partition to finish a tile sums it inside the launch, in the same order.
+  // The workspace is held for both, so that what may follow under capture does not depend on the way.
   const uint32_t kt = (k + cfg.tile_k - 1) / cfg.tile_k;
   p.k_per_split = ((kt + sk - 1) / sk) * cfg.tile_k;
+  const size_t slots = (size_t)p.tiles_m * p.tiles_n * sk * cfg.tile_m * cfg.tile_n * 4;
+  XcdExchange xk;
+  bool ok = false;
+  if (e->fn_exchange && !fixed && sk == 2 && slots <= kExchangeSlotBytes &&
+      xk_prepare(ctx, p.tiles_m * p.tiles_n, kExchangeSlotBytes, &xk, &ok) == T0MI_OK && ok) {
+    p.y = (void*)y;
+    return launch_gemm(ctx, cfg, e, p, &xk);
+  }
   p.y = ws;
   p.ldy = n;
   p.y_split_stride = plane;
