@@ -489,9 +489,11 @@ __device__ __forceinline__ bool exchange_partitions(f32x16 (&acc)[FN][FM], const
 }
 
 // One output tile (tm, tn) of K partition `part`: the whole kernel body, called
-// once by gemm_bf16_kernel and in a loop by the persistent kernel.  XK: the two partitions of a
-// tile are summed through `xk` (p.y, p.ldy: the final output); otherwise each partition stores its plane.
-template <int BM, int BN, int BK, int WM, int WN, int S, bool NN, bool XK = false>
+// once by gemm_bf16_kernel and in a loop by the persistent kernel.  SUMS: what becomes of
+// the sums: final or a plane (by p.split_k); a plane always; or the two partitions of a tile summed
+// through `xk` (p.y, p.ldy: the final output).
+enum TileSums { kSumsAny, kSumsPlane, kSumsExchange };
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN, TileSums SUMS = kSumsAny>
 __device__ __forceinline__ void gemm_bf16_tile(const GemmParams& p, int tm, int tn, int part,
                                                const XcdExchange* xk = nullptr) {
   using T = GemmTile<BM, BN, BK, WM, WN, S, NN>;
@@ -834,12 +836,17 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmParams& p, int tm, int 
   // i.e. four consecutive columns per (lane, g): one 16-byte (f32) or
   // 8-byte (bf16) store.  The (fm, fn) loops are expanded at compile time so
   // acc is only ever indexed by constants and stays in registers.
-  if constexpr (XK) {
+  if constexpr (SUMS == kSumsPlane) {
+    store_blocks<FM, FN, false>(p, acc, (char*)p.y + (size_t)part * p.y_split_stride, m0 + wm * TM, n0 + wn * TN, lane,
+                                true);
+    return;
+  }
+  if constexpr (SUMS == kSumsExchange) {
     if (!exchange_partitions<FM, FN, T::NTHR>(acc, *xk, (uint32_t)tm + (uint32_t)tn * p.tiles_m, (uint32_t)part,
                                               m0 + wm * TM + (lane & 31), (int)p.M))
       return;
   }
-  const bool partial_plane = !XK && p.split_k > 1;
+  const bool partial_plane = SUMS == kSumsAny && p.split_k > 1;
   char* ybase = (char*)p.y + (partial_plane ? (size_t)part * p.y_split_stride : 0);
   // Full tiles with bf16 output: stage each wave's block through the (now
   // idle) LDS ring and store whole rows, when the blocks fit in it.
@@ -866,7 +873,15 @@ template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_exchange_kernel(GemmParams p, XcdExchange xk) {
   int tm, tn, part;
   tile_coords(p, tm, tn, part);
-  gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, true>(p, tm, tn, part, &xk);
+  gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, kSumsExchange>(p, tm, tn, part, &xk);
+}
+
+// Planes only, without the epilogue's code.
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_planes_kernel(GemmParams p) {
+  int tm, tn, part;
+  tile_coords(p, tm, tn, part);
+  gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, kSumsPlane>(p, tm, tn, part);
 }
 
 }  // namespace t0mi

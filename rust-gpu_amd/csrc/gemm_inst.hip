@@ -23,6 +23,14 @@ static void launch_variant(dim3 g, hipStream_t s, const GemmParams& p) {
       return;
     }
   }
+  // Split-K of the tiles that the ranked schedule splits: a kernel without the epilogue's code
+  // (128x4096x4096, 64x128 in 4 parts: 14.0-14.3 us with it in the kernel, 13.9 without).
+  if constexpr (BM * BN <= 128 * 128 && BK == 64 && WM * WN == 4 && S >= 3) {
+    if (p.split_k > 1) {
+      hipLaunchKernelGGL((gemm_bf16_planes_kernel<BM, BN, BK, WM, WN, S, NN>), g, dim3(WM * WN * 64), 0, s, p);
+      return;
+    }
+  }
   hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, BK, WM, WN, S, NN>), g, dim3(WM * WN * 64), 0, s, p);
 }
 
