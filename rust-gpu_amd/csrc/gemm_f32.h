@@ -28,16 +28,16 @@
 //   * A tile that would end past the matrix starts earlier instead (it overlaps its neighbour,
 //     whose rows and columns it does not store), so no load needs a column mask.
 //
-// What bounds it: the CU's load path.  A K tile's f32 pieces enter a CU at 75-85 GB/s whatever the
+// What bounds it: the CU's load path.  A further K tile's f32 pieces enter a CU at 107-112 GB/s whatever the
 // tile and however many are in flight (two K tiles per group or four: the same times), so the time
 // is the operand bytes per CU, (bm + bn) * 4 * K for each of its tiles, over that rate, plus about
 // 4 us; hence larger tiles as soon as they still give every CU one, and K cut over workgroups where
 // they do not.  Large products pay that twice over (f32 pieces are twice the bf16 bytes, read once
 // per tile row and column), and the conversion passes win: f32_plan (gemm_f32_plan.h) draws the line.
 // Measured, forward + data + weight of one layer, before (conversion passes, GEMM, reduce, unpad) and
-// now: 512 tokens, 1024 -> 4096: 66.8 -> 49.8 us; 333 tokens, 1100 -> 770: 56.1 -> 29.8 us; forward
-// alone, 16 x 4096 x 4096: 27.9 -> 17.4 us; inference layer, 7 x 11008 x 2048: 12.7 -> 10.6 us.  The error against 64-bit sums is the smaller one
-// (1.9e-7 -> 1.3e-7 relative on the first): K is summed in chains of at most 1024.
+// now: 512 tokens, 1024 -> 4096: 66.8 -> 49.2 us; 333 tokens, 1100 -> 770: 56.1 -> 29.6 us; forward
+// alone, 16 x 4096 x 4096: 27.9 -> 17.2 us; inference layer, 7 x 11008 x 2048: 12.7 -> 10.6 us.  The
+// error against 64-bit sums is the smaller one (1.9e-7 -> 1.2e-7 relative on the first): K is summed in chains of at most 1024.
 #pragma once
 #include <type_traits>
 

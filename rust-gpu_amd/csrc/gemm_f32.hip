@@ -61,9 +61,12 @@ bool set_up(t0mi_ctx* ctx, const F32Plan& plan, int b_size, uint64_t a, uint64_t
   p->tiles_n = plan.tiles_n;
   p->pieces = plan.pieces;
   *grid = plan.tiles_m * plan.tiles_n;
+  // The slots are made by the first call of this route, split or not: what a later call may do under
+  // capture depends on a call before it, not on that call's sizes.
+  bool ok = false;
+  const bool exchange = xk_prepare(ctx, *grid, kF32SlotBytes, &p->x, &ok) == T0MI_OK && ok;
   if (plan.pieces > 1) {
-    bool ok = false;
-    if (xk_prepare(ctx, *grid, kF32SlotBytes, &p->x, &ok) != T0MI_OK || !ok) return false;
+    if (!exchange) return false;
     *grid = (*grid + p->x.nx - 1) / p->x.nx * p->x.nx * plan.pieces;
   }
   return true;

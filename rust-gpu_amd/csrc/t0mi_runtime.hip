@@ -1183,7 +1183,7 @@ extern "C" int t0mi_auto_gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t 
 // open, and its tile is one of an RDNA part's (64 x 64 x 16 on one wave, say), so the schedule that
 // auto_select ranks first for the shape runs under the spec's name, kernargs and grid, as for the
 // persistent presets (1000 x 2752 x 2056 NT, bias + GELU, bf16 out, tile_auto_select's 64x64 k16: 63.8
-// us on its own tile, 35.2 so).  The spec's tile remains for specs that name their split-K, for
+// us on its own tile, 24.1 so).  The spec's tile remains for specs that name their split-K, for
 // calls whose arguments are refused (it reports them), and where the schedule's split-K planes would
 // need workspace that may not grow now (a capture, or live graphs holding its address).
 static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e,
