@@ -39,15 +39,13 @@ void launch_wt(int tile, const GemmF32Params& p, uint32_t grid, hipStream_t s) {
                        dim3(512), 0, s, p);
 }
 
-bool overlap(uint64_t a, uint64_t an, uint64_t b, uint64_t bn) { return a < b + bn && b < a + an; }
-
 // Fills the parameters of a planned call and *grid.  False: the call takes the other route (an operand
 // overlaps Y, which that route reads whole before Y is written; or the exchange may not grow now).
 bool set_up(t0mi_ctx* ctx, const F32Plan& plan, int b_size, uint64_t a, uint64_t b, uint64_t y, uint32_t m, uint32_t n,
             uint32_t k, GemmF32Params* p, uint32_t* grid) {
   if (plan.tile < 0) return false;
   const uint64_t a_bytes = (uint64_t)m * k * 4, b_bytes = (uint64_t)k * n * b_size, y_bytes = (uint64_t)m * n * 4;
-  if (overlap(a, a_bytes, y, y_bytes) || overlap(b, b_bytes, y, y_bytes)) return false;
+  if (ranges_meet(a, a_bytes, y, y_bytes) || ranges_meet(b, b_bytes, y, y_bytes)) return false;
   memset(p, 0, sizeof *p);
   p->a = (const float*)a;
   p->b = (const void*)b;

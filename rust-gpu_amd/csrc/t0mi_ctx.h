@@ -187,6 +187,8 @@ struct FixedWorkspace {
 int run_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e, uint64_t x, uint64_t b,
              uint64_t y, uint64_t bias, uint32_t m, uint32_t n, uint32_t k, const EpiChain& epi,
              const FixedWorkspace* fixed = nullptr, uint32_t ldn = 0);
+// Whether [a, a + an) and [b, b + bn) meet.
+inline bool ranges_meet(uint64_t a, uint64_t an, uint64_t b, uint64_t bn) { return a < b + bn && b < a + an; }
 // True when the chain contains `op`.
 inline bool chain_uses(const EpiChain& e, uint32_t op) {
   for (uint32_t i = 0; i < e.n; ++i)

@@ -940,6 +940,15 @@ extern "C" int t0mi_wait_idle(t0mi_ctx* ctx) {
 // ---------------------------------------------------------- one-call GEMM ----
 
 namespace t0mi {
+// Whether the bytes of Y[m,n] meet those of X, B or the bias (row length ld of Y and of NN's B).
+static bool output_meets_operands(const t0mi_gemm_config& cfg, uint64_t x, uint64_t b, uint64_t y, uint64_t bias,
+                                  uint32_t m, uint32_t n, uint32_t k, uint32_t ld) {
+  const uint64_t y_bytes = ((uint64_t)(m - 1) * ld + n) * (cfg.out_dtype == T0MI_OUT_BF16 ? 2 : 4);
+  const uint64_t b_bytes = (cfg.transpose == T0MI_NN ? (uint64_t)(k - 1) * ld + n : (uint64_t)n * k) * 2;
+  return ranges_meet(x, (uint64_t)m * k * 2, y, y_bytes) || ranges_meet(b, b_bytes, y, y_bytes) ||
+         (bias && ranges_meet(bias, (uint64_t)n * 4, y, y_bytes));
+}
+
 int run_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e, uint64_t x, uint64_t b,
              uint64_t y, uint64_t bias, uint32_t m, uint32_t n, uint32_t k, const EpiChain& epi,
              const FixedWorkspace* fixed, uint32_t ldn) {
@@ -1003,6 +1012,8 @@ int run_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* 
   // Split-K: partitions of whole K tiles write f32 planes into the workspace,
   // then a reduce pass sums them in partition order; or, where that is faster (exchange_of in
   // gemm_inst.hip), the last partition to finish a tile sums it inside the launch, in the same order.
+  // Planes also where Y lies over an operand: the reduce writes Y after the last read of the operands, the
+  // exchange stores a tile while other tiles still read theirs.
   // The workspace is held for both, so that what may follow under capture does not depend on the way.
   const uint32_t kt = (k + cfg.tile_k - 1) / cfg.tile_k;
   p.k_per_split = ((kt + sk - 1) / sk) * cfg.tile_k;
@@ -1010,6 +1021,7 @@ int run_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* 
   XcdExchange xk;
   bool ok = false;
   if (e->fn_exchange && !fixed && sk == 2 && slots <= kExchangeSlotBytes &&
+      !output_meets_operands(cfg, x, b, y, bias, m, n, k, ld) &&
       xk_prepare(ctx, p.tiles_m * p.tiles_n, kExchangeSlotBytes, &xk, &ok) == T0MI_OK && ok) {
     p.y = (void*)y;
     return launch_gemm(ctx, cfg, e, p, &xk);

@@ -61,6 +61,31 @@ def test_equals_planes(rt, m, n, k, nn, od, epilogue, stages):
     assert (np.abs(got - exact) <= lim).all()
 
 
+@pytest.mark.parametrize("m,n,k", [(128, 1024, 1024), (100, 1032, 1032)])
+@pytest.mark.parametrize("over", ["x", "b", "bias"])
+@pytest.mark.parametrize("nn", [False, True])
+def test_output_over_an_operand(rt, m, n, k, over, nn):
+    """Y (bf16) in an operand's place, with the configuration the ranking picks: the planes route, whose
+    reduce runs after the last read of the operands, as gemm_noalloc."""
+    cfg = t0mi.auto_select_layout(m, k, n, t0mi.NN if nn else t0mi.NT, t0mi.OUT_BF16)
+    assert (cfg.tile_m, cfg.tile_n, cfg.split_k) == (64, 64, 2)
+    cfg = cfg.copy(epilogue=t0mi.EPI_BIAS_ADD)
+    a = oracle.normal_bf16((m, k), m + k, 0.0, 1.0)
+    b = oracle.normal_bf16((k, n) if nn else (n, k), n + k, 0.0, 1.0)
+    bias = np.linspace(-1, 1, n, dtype=np.float32)
+
+    def call(f, y):
+        ops = {"x": a, "b": b, "bias": np.concatenate([bias, np.zeros(m * n // 2, np.float32)])}
+        dev = {o: to_dev(v) for o, v in ops.items()}
+        dy, py = dev[y] if y else empty_dev(m * n * 2, fill=0xCD)
+        f(cfg, dev["x"][1], dev["b"][1], py, m, n, k, dev["bias"][1])
+        return from_dev(dy, np.uint16, (m, n))
+
+    want = call(rt.gemm_noalloc, None)
+    for _ in range(3):
+        assert np.array_equal(call(rt.gemm, over), want)
+
+
 def test_capture(rt):
     th = torch()
     st = th.cuda.Stream()
