@@ -351,9 +351,19 @@ extern "C" int t0mi_gptq_convert(t0mi_ctx* ctx, uint64_t packed, uint64_t scales
   const uint64_t q_wgs = (uint64_t)((K8 + 63) / 64) * ((rows + 63) / 64);
   const uint64_t p_wgs =
       (uint64_t)((G + kGptqTileG - 1) / kGptqTileG) * ((rows + kGptqTileN - 1) / kGptqTileN);
-  hipLaunchKernelGGL(gptq_convert_kernel, dim3((uint32_t)(q_wgs + p_wgs)), dim3(256), 0, ctx->stream,
-                     (const uint32_t*)packed, (const float*)scales_f32, (const int32_t*)zeros_i32, (uint32_t*)qweight,
-                     (uint16_t*)scales_bf16, (uint32_t*)qzeros, rows, K8, G, (uint32_t)p_wgs);
-  const hipError_t e = hipGetLastError();
-  return e == hipSuccess ? T0MI_OK : hip_fail(e, "gptq conversion launch");
+  // One launch for both parts; or the weights first, where a parameter output lies over the packed words
+  // they are read from.
+  const auto launch = [&](uint64_t wgs, uint64_t params) {
+    hipLaunchKernelGGL(gptq_convert_kernel, dim3((uint32_t)wgs), dim3(256), 0, ctx->stream, (const uint32_t*)packed,
+                       (const float*)scales_f32, (const int32_t*)zeros_i32, (uint32_t*)qweight,
+                       (uint16_t*)scales_bf16, (uint32_t*)qzeros, rows, K8, G, (uint32_t)params);
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? T0MI_OK : hip_fail(e, "gptq conversion launch");
+  };
+  const uint64_t packed_bytes = (uint64_t)rows * K8 * 4, params = (uint64_t)G * rows;
+  if (!ranges_meet(packed, packed_bytes, scales_bf16, params * 2) &&
+      !ranges_meet(packed, packed_bytes, qzeros, params / 2))
+    return launch(q_wgs + p_wgs, p_wgs);
+  if (int rc = launch(q_wgs, 0)) return rc;
+  return launch(p_wgs, p_wgs);
 }

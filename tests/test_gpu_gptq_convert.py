@@ -57,3 +57,23 @@ def test_gptq_convert(rt, rows, cols, group, off):
     assert np.array_equal(got[0].view(np.uint32).reshape(cols // 8, rows), oracle.pack_qweight(q))
     assert np.array_equal(got[1].view(np.uint16).reshape(ng, rows), oracle.bf16_rne(np.ascontiguousarray(scales.T)))
     assert np.array_equal(got[2].view(np.uint32).reshape(ng, rows // 8), oracle.pack_qzeros(zeros))
+
+
+@pytest.mark.parametrize("rows,cols,group", [(72, 520, 8), (4096, 2048, 128)])
+def test_parameters_over_the_packed_weights(rt, rows, cols, group):
+    """scales_bf16 and qzeros in the packed buffer, whose words are no longer needed."""
+    q, scales, zeros = case(rows, cols, group, rows + cols)
+    ng = cols // group
+    dp, pp = to_dev(np.ascontiguousarray(oracle.pack_gptq_bytes(q)))
+    ds, ps = to_dev(scales)
+    dz, pz = to_dev(np.ascontiguousarray(zeros.T.astype(np.int32)))
+    dq, pq = empty_dev(cols // 8 * rows * 4, fill=0xAA)
+    sb, zb = ng * rows * 2, ng * rows // 2
+    rt.gptq_convert(pp, ps, pz, rows, cols, group, pq, pp, pp + sb)
+    torch().cuda.synchronize()
+    check_guard(dq)
+    b = dp[:sb + zb].cpu().numpy()
+    assert np.array_equal(dq[:cols // 8 * rows * 4].cpu().numpy().view(np.uint32).reshape(cols // 8, rows),
+                          oracle.pack_qweight(q))
+    assert np.array_equal(b[:sb].view(np.uint16).reshape(ng, rows), oracle.bf16_rne(np.ascontiguousarray(scales.T)))
+    assert np.array_equal(b[sb:].view(np.uint32).reshape(ng, rows // 8), oracle.pack_qzeros(zeros))

@@ -31,3 +31,22 @@ done(dict(
 """)
     assert all(c == ["gemm_bf16_exchange_kernel"] for c in r["apart"]), r["apart"]
     assert all(c == PLANES for c in r["over"]), r["over"]
+
+
+def test_gptq_parameters_over_the_packed_weights(host):
+    """The weights are read whole before scales or zero points are written into their place."""
+    r = host("""
+rows, cols, group = 72, 520, 8
+pk, pr = rows * cols // 2, cols // group * rows
+S, Z, Q, S2, Z2 = [i << 40 for i in range(2, 7)]
+hip.fake_launches()
+def grids(s2, z2):
+    rt.gptq_convert(X, S, Z, rows, cols, group, Q, s2, z2)
+    return [l[1] for l in launches()]
+done(dict(apart=[grids(S2, Z2), grids(X + pk, Z2), grids(S2, X + pk), grids(X - pr * 2, Z2), grids(S2, X - pr // 2)],
+          over=[grids(X, Z2), grids(S2, X), grids(X + pk - 2, Z2), grids(X - pr * 2 + 2, Z2), grids(S2, X + pk - 4),
+                grids(S2, X - pr // 2 + 4), grids(X, X + pr * 2)]))
+""")
+    weights, params = 2 * 2, 3 * 2  # 65 words and 72 rows in 64s; 65 groups in 32s and 72 rows in 64s
+    assert r["apart"] == [[weights + params]] * 5
+    assert r["over"] == [[weights, params]] * 7
