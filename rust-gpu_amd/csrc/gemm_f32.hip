@@ -39,13 +39,13 @@ void launch_wt(int tile, const GemmF32Params& p, uint32_t grid, hipStream_t s) {
                        dim3(512), 0, s, p);
 }
 
-// Fills the parameters of a planned call and *grid.  False: the call takes the other route (an operand
-// overlaps Y, which that route reads whole before Y is written; or the exchange may not grow now).
-bool set_up(t0mi_ctx* ctx, const F32Plan& plan, int b_size, uint64_t a, uint64_t b, uint64_t y, uint32_t m, uint32_t n,
-            uint32_t k, GemmF32Params* p, uint32_t* grid) {
-  if (plan.tile < 0) return false;
+// Fills the parameters of a planned call and *grid.  1: the call takes the other route (an operand
+// overlaps Y, which that route reads whole before Y is written; or the exchange cannot be had now).
+int set_up(t0mi_ctx* ctx, const F32Plan& plan, int b_size, uint64_t a, uint64_t b, uint64_t y, uint32_t m, uint32_t n,
+           uint32_t k, GemmF32Params* p, uint32_t* grid) {
+  if (plan.tile < 0) return 1;
   const uint64_t a_bytes = (uint64_t)m * k * 4, b_bytes = (uint64_t)k * n * b_size, y_bytes = (uint64_t)m * n * 4;
-  if (ranges_meet(a, a_bytes, y, y_bytes) || ranges_meet(b, b_bytes, y, y_bytes)) return false;
+  if (ranges_meet(a, a_bytes, y, y_bytes) || ranges_meet(b, b_bytes, y, y_bytes)) return 1;
   memset(p, 0, sizeof *p);
   p->a = (const float*)a;
   p->b = (const void*)b;
@@ -62,12 +62,12 @@ bool set_up(t0mi_ctx* ctx, const F32Plan& plan, int b_size, uint64_t a, uint64_t
   // The slots are made by the first call of this route, split or not: what a later call may do under
   // capture depends on a call before it, not on that call's sizes.
   bool ok = false;
-  const bool exchange = xk_prepare(ctx, *grid, kF32SlotBytes, &p->x, &ok) == T0MI_OK && ok;
+  if (int rc = xk_prepare(ctx, *grid, kF32SlotBytes, &p->x, &ok, true)) return rc;
   if (plan.pieces > 1) {
-    if (!exchange) return false;
+    if (!ok) return 1;
     *grid = (*grid + p->x.nx - 1) / p->x.nx * p->x.nx * plan.pieces;
   }
-  return true;
+  return T0MI_OK;
 }
 
 int launched() {
@@ -82,7 +82,7 @@ int run_gemm_f32(t0mi_ctx* ctx, int mode, uint64_t a, uint64_t b, uint64_t y, ui
   const F32Plan plan = f32_plan(mode, m, n, k, (uint32_t)ctx->cu_count, ctx->xk_nx > 0);
   GemmF32Params p;
   uint32_t grid;
-  if (!set_up(ctx, plan, 4, a, b, y, m, n, k, &p, &grid)) return 1;
+  if (int rc = set_up(ctx, plan, 4, a, b, y, m, n, k, &p, &grid)) return rc;
   p.lda = f32_a_kmajor(mode) ? m : k;
   p.ldb = f32_b_kmajor(mode) ? n : k;
   switch (mode) {
@@ -98,7 +98,7 @@ int run_gemm_wt(t0mi_ctx* ctx, uint64_t x, uint64_t wt, uint64_t y, uint32_t m, 
   const F32Plan plan = wt_plan(m, n, k, (uint32_t)ctx->cu_count, ctx->xk_nx > 0);
   GemmF32Params p;
   uint32_t grid;
-  if (!set_up(ctx, plan, 2, x, wt, y, m, n, k, &p, &grid)) return 1;
+  if (int rc = set_up(ctx, plan, 2, x, wt, y, m, n, k, &p, &grid)) return rc;
   p.lda = k;
   p.ldb = k;
   launch_wt(plan.tile, p, grid, ctx->stream);

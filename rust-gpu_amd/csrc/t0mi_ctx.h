@@ -111,8 +111,9 @@ struct t0mi_ctx {
 namespace t0mi {
 // Grows ctx->ws to at least `bytes` (waits for the stream first).
 int ensure_workspace(t0mi_ctx* ctx, size_t bytes);
-// Whether ctx->ws holds `bytes` or may grow to (no capture, no live graph holding its address).
-bool workspace_available(t0mi_ctx* ctx, size_t bytes);
+// The same for a route that another one can stand in for: *ok is false, and no error is set, where the
+// workspace may not grow now (a capture, live graphs holding its address) or memory is out.
+int try_workspace(t0mi_ctx* ctx, size_t bytes, bool* ok);
 // Grows ctx->cvt to at least `bytes` (waits for the stream first).
 int ensure_cvt_buffer(t0mi_ctx* ctx, size_t bytes);
 // Counters of the XCD exchange, per XCD: at most this many tiles per XCD per launch.
@@ -126,8 +127,8 @@ constexpr size_t kExchangeSlotBytes = 32u << 20;
 // Readies the XCD exchange for a launch of `tiles` tiles with `part_bytes` of
 // partial slots: false (no error set) when the device's placement did not
 // check out or the tiles do not fit the counters; T0MI_ERR_* when a buffer
-// could not be made.  Fills *x.
-int xk_prepare(t0mi_ctx* ctx, uint32_t tiles, size_t part_bytes, XcdExchange* x, bool* ok);
+// could not be made (`optional`: false as well, as try_workspace).  Fills *x.
+int xk_prepare(t0mi_ctx* ctx, uint32_t tiles, size_t part_bytes, XcdExchange* x, bool* ok, bool optional = false);
 // Runs a GEMM with the best prebuilt config for (m, n, k, transpose) and the
 // given output type (cost-model ranking, as t0mi_auto_select), as two launches
 // over column ranges where plan_column_split says so; NT calls of up to 16 rows

@@ -89,6 +89,15 @@ int fill_async(t0mi_ctx* ctx, void* dst, uint8_t value, size_t bytes) {
   return e == hipSuccess ? T0MI_OK : hip_fail(e, "fill launch");
 }
 
+// Whether ctx's stream is being captured (no error is set; a failed query counts as a capture).
+static bool capturing(t0mi_ctx* ctx) {
+  if (ctx->null_backend || !ctx->stream) return false;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // A buffer that graphs still reference cannot be replaced; one that must grow
 // while the stream is captured cannot be allocated (run the work once eagerly
 // first: the buffers only grow, so a captured replay then fits).
@@ -105,74 +114,81 @@ static int check_growth(t0mi_ctx* ctx, const char* what, size_t have, size_t wan
   return rc;
 }
 
-int ensure_workspace(t0mi_ctx* ctx, size_t bytes) {
-  if (ctx->ws_bytes >= bytes) return T0MI_OK;
+// Grows *buf (*have bytes) to `bytes` and some slack.  With `ok` the caller can do without: where the
+// buffer may not grow now or memory is out, *ok is false, the old buffer stays and no error is left
+// behind, in the library's text or in HIP's last error, which the next launch check would report.
+static int grow(t0mi_ctx* ctx, const char* what, void** buf, size_t* have, size_t bytes, bool* ok = nullptr) {
+  if (ok) *ok = true;
+  if (*have >= bytes) return T0MI_OK;
   if (ctx->null_backend) {
-    ctx->ws_bytes = bytes;
+    *have = bytes;
     return T0MI_OK;
   }
-  if (int rc = check_growth(ctx, "the split-K workspace", ctx->ws_bytes, bytes)) return rc;
+  if (ok) {
+    *ok = ctx->live_graphs.load() == 0 && !capturing(ctx);
+    if (!*ok) return T0MI_OK;
+  } else if (int rc = check_growth(ctx, what, *have, bytes)) {
+    return rc;
+  }
   hipError_t e = hipStreamSynchronize(ctx->stream);
   if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
-  if (ctx->ws) (void)hipFree(ctx->ws);
-  ctx->ws = nullptr;
-  ctx->ws_bytes = 0;
-  size_t want = bytes + (bytes >> 2);  // grow with slack
-  e = hipMalloc(&ctx->ws, want);
-  if (e != hipSuccess) return hip_fail(e, "hipMalloc(workspace)");
-  ctx->ws_bytes = want;
+  if (!ok) {
+    if (*buf) (void)hipFree(*buf);
+    *buf = nullptr;
+    *have = 0;
+  }
+  const size_t want = bytes + (bytes >> 2);
+  void* p = nullptr;
+  e = hipMalloc(&p, want);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    if (!ok) return hip_fail(e, what);
+    *ok = false;
+    return T0MI_OK;
+  }
+  if (*buf) (void)hipFree(*buf);
+  *buf = p;
+  *have = want;
   return T0MI_OK;
 }
 
-bool workspace_available(t0mi_ctx* ctx, size_t bytes) {
-  return bytes <= ctx->ws_bytes ||
-         (ctx->live_graphs.load() == 0 && refuse_if_capturing(ctx, "growing the library workspace") == T0MI_OK);
+int ensure_workspace(t0mi_ctx* ctx, size_t bytes) {
+  return grow(ctx, "the split-K workspace", &ctx->ws, &ctx->ws_bytes, bytes);
+}
+
+int try_workspace(t0mi_ctx* ctx, size_t bytes, bool* ok) {
+  return grow(ctx, "the split-K workspace", &ctx->ws, &ctx->ws_bytes, bytes, ok);
 }
 
 int ensure_cvt_buffer(t0mi_ctx* ctx, size_t bytes) {
-  if (ctx->cvt_bytes >= bytes) return T0MI_OK;
-  if (ctx->null_backend) {
-    ctx->cvt_bytes = bytes;
-    return T0MI_OK;
-  }
-  if (int rc = check_growth(ctx, "the conversion buffer", ctx->cvt_bytes, bytes)) return rc;
-  hipError_t e = hipStreamSynchronize(ctx->stream);
-  if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
-  if (ctx->cvt) (void)hipFree(ctx->cvt);
-  ctx->cvt = nullptr;
-  ctx->cvt_bytes = 0;
-  size_t want = bytes + (bytes >> 2);
-  e = hipMalloc(&ctx->cvt, want);
-  if (e != hipSuccess) return hip_fail(e, "hipMalloc(conversion buffer)");
-  ctx->cvt_bytes = want;
-  return T0MI_OK;
+  return grow(ctx, "the conversion buffer", &ctx->cvt, &ctx->cvt_bytes, bytes);
 }
 
-int xk_prepare(t0mi_ctx* ctx, uint32_t tiles, size_t part_bytes, XcdExchange* x, bool* ok) {
+int xk_prepare(t0mi_ctx* ctx, uint32_t tiles, size_t part_bytes, XcdExchange* x, bool* ok, bool optional) {
   *ok = false;
   if (ctx->null_backend || ctx->xk_nx == 0) return T0MI_OK;
   if ((tiles + ctx->xk_nx - 1) / ctx->xk_nx > kXkCountersPerXcd) return T0MI_OK;
-  const size_t tick_bytes = ((size_t)ctx->xk_nx * kXkCountersPerXcd + 1) * kXkCounterStride * 4;  // + the flag
+  bool fits = true;
+  bool* const may_fail = optional ? &fits : nullptr;
   if (!ctx->xk_tick) {
-    if (int rc = check_growth(ctx, "the exchange counters", 0, tick_bytes)) return rc;
-    hipError_t e = hipMalloc((void**)&ctx->xk_tick, tick_bytes);
-    if (e != hipSuccess) return hip_fail(e, "hipMalloc(exchange counters)");
-    if (int rc = fill_async(ctx, ctx->xk_tick, 0, tick_bytes)) return rc;
-    e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
+    const size_t tick_bytes = ((size_t)ctx->xk_nx * kXkCountersPerXcd + 1) * kXkCounterStride * 4;  // + the flag
+    void* tick = nullptr;
+    size_t have = 0;
+    if (int rc = grow(ctx, "the exchange counters", &tick, &have, tick_bytes, may_fail)) return rc;
+    if (!fits) return T0MI_OK;
+    int rc = fill_async(ctx, tick, 0, tick_bytes);
+    if (rc == T0MI_OK) {
+      const hipError_t e = hipStreamSynchronize(ctx->stream);
+      if (e != hipSuccess) rc = hip_fail(e, "hipStreamSynchronize");
+    }
+    if (rc) {
+      (void)hipFree(tick);
+      return rc;
+    }
+    ctx->xk_tick = (uint32_t*)tick;
   }
-  if (ctx->xk_part_bytes < part_bytes) {
-    if (int rc = check_growth(ctx, "the exchange slots", ctx->xk_part_bytes, part_bytes)) return rc;
-    hipError_t e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
-    if (ctx->xk_part) (void)hipFree(ctx->xk_part);
-    ctx->xk_part = nullptr;
-    ctx->xk_part_bytes = 0;
-    const size_t want = part_bytes + (part_bytes >> 2);
-    e = hipMalloc(&ctx->xk_part, want);
-    if (e != hipSuccess) return hip_fail(e, "hipMalloc(exchange slots)");
-    ctx->xk_part_bytes = want;
-  }
+  if (int rc = grow(ctx, "the exchange slots", &ctx->xk_part, &ctx->xk_part_bytes, part_bytes, may_fail)) return rc;
+  if (!fits) return T0MI_OK;
   x->part = (float*)ctx->xk_part;
   x->tick = ctx->xk_tick;
   x->flag = ctx->xk_tick + (size_t)ctx->xk_nx * kXkCountersPerXcd * kXkCounterStride;
@@ -1018,13 +1034,16 @@ int run_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* 
   const uint32_t kt = (k + cfg.tile_k - 1) / cfg.tile_k;
   p.k_per_split = ((kt + sk - 1) / sk) * cfg.tile_k;
   const size_t slots = (size_t)p.tiles_m * p.tiles_n * sk * cfg.tile_m * cfg.tile_n * 4;
-  XcdExchange xk;
-  bool ok = false;
   if (e->fn_exchange && !fixed && sk == 2 && slots <= kExchangeSlotBytes &&
-      !output_meets_operands(cfg, x, b, y, bias, m, n, k, ld) &&
-      xk_prepare(ctx, p.tiles_m * p.tiles_n, kExchangeSlotBytes, &xk, &ok) == T0MI_OK && ok) {
-    p.y = (void*)y;
-    return launch_gemm(ctx, cfg, e, p, &xk);
+      !output_meets_operands(cfg, x, b, y, bias, m, n, k, ld)) {
+    XcdExchange xk;
+    bool ok = false;
+    rc = xk_prepare(ctx, p.tiles_m * p.tiles_n, kExchangeSlotBytes, &xk, &ok, true);
+    if (rc) return rc;
+    if (ok) {
+      p.y = (void*)y;
+      return launch_gemm(ctx, cfg, e, p, &xk);
+    }
   }
   p.y = ws;
   p.ldy = n;
@@ -1197,7 +1216,7 @@ extern "C" int t0mi_auto_gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t 
 // persistent presets (1000 x 2752 x 2056 NT, bias + GELU, bf16 out, tile_auto_select's 64x64 k16: 63.8
 // us on its own tile, 24.1 so).  The spec's tile remains for specs that name their split-K, for
 // calls whose arguments are refused (it reports them), and where the schedule's split-K planes would
-// need workspace that may not grow now (a capture, or live graphs holding its address).
+// need workspace that cannot be had now (a capture, live graphs holding its address, no memory left).
 static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e,
                          uint64_t x, uint64_t b, uint64_t y, uint64_t bias, uint32_t m, uint32_t n, uint32_t k,
                          const EpiChain& chain) {
@@ -1208,8 +1227,9 @@ static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm
       cached_auto_plan(m, n, k, cfg.transpose, cfg.out_dtype, (uint32_t)ctx->cu_count, &pl)) {
     const uint32_t sk_h = split_k_of(pl.head), sk_t = pl.n1 < n ? split_k_of(pl.tail) : 1;
     const size_t need = std::max(sk_h > 1 ? (size_t)m * pl.n1 * 4 * sk_h : 0, sk_t > 1 ? (size_t)m * (n - pl.n1) * 4 * sk_t : 0);
-    if (workspace_available(ctx, need))
-      return run_gemm_auto(ctx, cfg.transpose, x, b, y, m, n, k, cfg.out_dtype, bias, &chain);
+    bool ok = false;
+    if (int rc = try_workspace(ctx, need, &ok)) return rc;
+    if (ok) return run_gemm_auto(ctx, cfg.transpose, x, b, y, m, n, k, cfg.out_dtype, bias, &chain);
   }
   return run_gemm(ctx, cfg, e, x, b, y, bias, m, n, k, chain);
 }

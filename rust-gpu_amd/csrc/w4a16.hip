@@ -694,9 +694,14 @@ extern "C" int t0mi_w4a16_gemm(t0mi_ctx* ctx, uint64_t a, uint64_t qweight, uint
   // launch (one pass over the weights feeds them all), spread evenly over the
   // fewest launches (5 slabs as 3 + 2, not 4 + 1); the other kernels one.
   const uint32_t slabs = (m + 15) / 16;
-  // Planes of every row (several tiles in one launch) only where the workspace may hold them now.
+  // Planes of every row (several tiles in one launch) only where the workspace can hold them now.
   uint32_t tile_rs = v2 ? decode_row_tiles(slabs, decode_max_slabs(group), strips * ky, (uint32_t)ctx->cu_count) : 0;
-  if (tile_rs && ky > 1 && !workspace_available(ctx, (size_t)m * n * 4 * ky)) tile_rs = 0;
+  if (tile_rs && ky > 1) {
+    bool ok = false;
+    rc = try_workspace(ctx, (size_t)m * n * 4 * ky, &ok);
+    if (rc) return rc;
+    if (!ok) tile_rs = 0;
+  }
   const uint32_t tiles = tile_rs ? (slabs + tile_rs - 1) / tile_rs : 1;
   const uint32_t launches = tile_rs ? 1 : v2 ? (slabs + decode_max_slabs(group) - 1) / decode_max_slabs(group) : slabs;
   for (uint32_t r0 = 0, done = 0, l = 0, rs = 1; r0 < m; r0 += 16 * rs * tiles, done += rs, ++l) {

@@ -50,3 +50,81 @@ done(dict(apart=[grids(S2, Z2), grids(X + pk, Z2), grids(S2, X + pk), grids(X - 
     weights, params = 2 * 2, 3 * 2  # 65 words and 72 rows in 64s; 65 groups in 32s and 72 rows in 64s
     assert r["apart"] == [[weights + params]] * 5
     assert r["over"] == [[weights, params]] * 7
+
+
+MEMORY = """
+def call(f, *args):
+    "The kernels of a call, its error text (None: it returned OK) and the library's text after it."
+    hip.fake_launches()
+    try:
+        f(*args)
+        e = None
+    except t0mi.T0miError as x:
+        e = str(x)
+    return [[l[0].split("<")[0] for l in launches()], e, t0mi.last_error()]
+cfg = t0mi.auto_select_layout(128, 1024, 1024, t0mi.NT, t0mi.OUT_BF16)
+spec = t0mi.tile_auto_select(128, 1024, 1024, t0mi.NT)
+calls = dict(
+    f32=lambda: call(rt.matmul, X, B, Y, 512, 1024, 517),        # one piece: needs no slots
+    f32_pieces=lambda: call(rt.matmul, X, B, Y, 40, 1000, 300),  # K pieces
+    gemm=lambda: call(rt.gemm, cfg, X, B, Y, 128, 1024, 1024),   # two K partitions
+    tile=lambda: call(rt.tile_gemm, spec, X, B, Y, 128, 1024, 1024),
+    w4=lambda: call(rt.w4a16_gemm, X, B, 5 << 40, 0, 8, Y, 100, 8192, 520, 128),  # K planes, row tiles
+)
+try:
+    rt.matmul(X + 4, B, Y, 8, 8, 8)
+except t0mi.T0miError:
+    pass
+before = t0mi.last_error()
+assert "aligned" in before
+"""
+
+
+def test_routes_with_memory(host):
+    r = host(MEMORY + "done({n: f() for n, f in calls.items()})")
+    assert {n: c[0] for n, c in r.items()} == {
+        "f32": ["t0mi_fill_kernel", "gemm_f32_kernel"],  # the exchange's counters are made by the first call
+        "f32_pieces": ["gemm_f32_kernel"],
+        "gemm": ["gemm_bf16_exchange_kernel"],
+        "tile": ["gemm_bf16_exchange_kernel"],
+        "w4": ["w4a16_decode_v2", "t0mi_splitk_reduce"],
+    }
+    assert all(c[1] is None for c in r.values())
+
+
+@pytest.mark.parametrize("limit", [8 << 20, 400 << 10])
+def test_no_memory_for_an_optional_buffer(host, limit):
+    """Out of memory for buffers that a call can do without: it takes its other route, or the same one if it
+    does not use them, returns OK, and leaves the library's error text as it was.  (HIP's last error, if
+    the failed allocation stayed in it, would fail the launch check.)"""
+    r = host(MEMORY + f"""
+rt.matmul(X, B, Y, 4096, 1024, 4096)  # makes the conversion passes' buffer
+if {limit} < 1 << 20:
+    del calls["gemm"]  # its partial planes have to fit
+hip.fake_set_malloc_limit({limit})
+out = {{n: f() for n, f in calls.items()}}
+done([before, out])
+""")
+    before, out = r
+    assert all(c[1] is None and c[2] == before for c in out.values()), out
+    assert out["f32"][0][-1] == "gemm_f32_kernel"
+    assert out["f32_pieces"][0] == ["cvt_bf16_kernel"] * 2 + out["f32_pieces"][0][2:]
+    if limit < 1 << 20:  # no workspace for planes either
+        assert out["tile"][0] == ["gemm_bf16_kernel"]
+        assert out["w4"][0] == ["w4a16_decode_v2", "t0mi_splitk_reduce"] * 2
+    else:
+        assert out["gemm"][0] == out["tile"][0] == PLANES
+
+
+def test_first_call_under_capture(host):
+    """Buffers that may not grow now: as above, and the captured calls return OK."""
+    r = host(MEMORY + """
+calls = {n: calls[n] for n in ("f32", "tile")}
+rt.capture_begin()
+out = {n: f() for n, f in calls.items()}
+rt.capture_end()
+done([before, out])
+""")
+    before, out = r
+    assert all(c[1] is None and c[2] == before for c in out.values()), out
+    assert out["f32"][0] == ["gemm_f32_kernel"] and out["tile"][0] == ["gemm_bf16_kernel"]
