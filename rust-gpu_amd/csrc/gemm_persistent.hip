@@ -142,10 +142,14 @@ int run_gemm_persistent(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLa
   return T0MI_OK;
 }
 
+bool gemm_decode_nt_takes(const t0mi_ctx* ctx, uint32_t m, uint32_t n, uint32_t k) {
+  if (m == 0 || m > 16 || k == 0 || k % 32 || n % 8 || (uint64_t)n > 16ull * (uint64_t)ctx->cu_count) return false;
+  return (uint64_t)m * k * 2 < (1ull << 32) && (uint64_t)n * k * 2 < (1ull << 32);
+}
+
 int run_gemm_decode_nt(t0mi_ctx* ctx, uint64_t x, uint64_t b, uint64_t y, uint32_t m, uint32_t n, uint32_t k,
                        uint32_t out_dtype, uint64_t bias, const EpiChain& epi) {
-  if (m == 0 || m > 16 || k == 0 || k % 32 || n % 8 || (uint64_t)n > 16ull * (uint64_t)ctx->cu_count) return 1;
-  if ((uint64_t)m * k * 2 >= (1ull << 32) || (uint64_t)n * k * 2 >= (1ull << 32)) return 1;
+  if (!gemm_decode_nt_takes(ctx, m, n, k)) return 1;
   // Argument errors are left to the caller's general route, which reports them.
   if ((x | b | y) & 15 || bias & 3 || (chain_uses(epi, EOP_BIAS) && !bias)) return 1;
   GemmParams p;

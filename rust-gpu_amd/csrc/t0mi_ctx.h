@@ -116,6 +116,8 @@ int ensure_workspace(t0mi_ctx* ctx, size_t bytes);
 int try_workspace(t0mi_ctx* ctx, size_t bytes, bool* ok);
 // Grows ctx->cvt to at least `bytes` (waits for the stream first).
 int ensure_cvt_buffer(t0mi_ctx* ctx, size_t bytes);
+// As try_workspace.
+int try_cvt_buffer(t0mi_ctx* ctx, size_t bytes, bool* ok);
 // Counters of the XCD exchange, per XCD: at most this many tiles per XCD per launch.
 // Each counter has a 256-byte slot of its own: atomics on one line (or one L2
 // channel) are serialized, and a launch's pieces all arrive at about the same
@@ -135,6 +137,9 @@ int xk_prepare(t0mi_ctx* ctx, uint32_t tiles, size_t part_bytes, XcdExchange* x,
 // run the persistent decode kernel instead (run_gemm_decode_nt).  Asynchronous.
 int run_gemm_auto(t0mi_ctx* ctx, uint32_t transpose, uint64_t x, uint64_t b, uint64_t y, uint32_t m, uint32_t n,
                   uint32_t k, uint32_t out_dtype = T0MI_OUT_F32, uint64_t bias = 0, const EpiChain* epi = nullptr);
+// Bytes of ctx->ws that run_gemm_auto needs for its partial planes.  False: no prebuilt kernel.
+bool gemm_auto_workspace(t0mi_ctx* ctx, uint32_t transpose, uint32_t m, uint32_t n, uint32_t k, uint32_t out_dtype,
+                         size_t* bytes);
 // The schedule of an auto-scheduled GEMM: the ranking's first config with a
 // prebuilt kernel over columns [0, n1) and, when n1 < n, the planned tail
 // config over [n1, n) (plan_column_split with `cus` compute units).  False
@@ -152,6 +157,7 @@ bool auto_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t transpose, uint32_t 
 // (gemm_persistent.hip), which beats the split-K schedule there (1 / 16 x 4096
 // x 4096, f32 out: 8.5 / 11.5 against 13.6 / 12.4 us).  Returns 1, launching
 // nothing, when the call is outside that range or its arguments are invalid.
+bool gemm_decode_nt_takes(const t0mi_ctx* ctx, uint32_t m, uint32_t n, uint32_t k);
 int run_gemm_decode_nt(t0mi_ctx* ctx, uint64_t x, uint64_t b, uint64_t y, uint32_t m, uint32_t n, uint32_t k,
                        uint32_t out_dtype, uint64_t bias, const EpiChain& epi);
 int run_gemm_planned(t0mi_ctx* ctx, const AutoPlan& pl, uint32_t transpose, uint64_t x, uint64_t b, uint64_t y,

@@ -239,6 +239,18 @@ int gemm_into(t0mi_ctx* ctx, uint32_t transpose, size_t b_off, uint64_t y, uint3
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
+// After a one-launch product: holds, as far as memory allows, what the conversion passes of the same call
+// would use (`cvt_bytes`, and the planes of their [m, k] x [k, n] GEMM).  Which of the two routes is the
+// faster is no matter of size alone (522 columns, K = 4230: passes up to 1599 rows, one launch at 1659),
+// and a program that runs its largest batch once may then capture smaller ones.
+int hold_passes(t0mi_ctx* ctx, size_t cvt_bytes, uint32_t transpose, uint32_t m, uint32_t n, uint32_t k) {
+  bool ok = false;
+  if (int rc = try_cvt_buffer(ctx, cvt_bytes, &ok)) return rc;
+  size_t planes = 0;
+  if (!ok || !gemm_auto_workspace(ctx, transpose, m, n, k, T0MI_OUT_F32, &planes)) return T0MI_OK;
+  return try_workspace(ctx, planes, &ok);
+}
+
 }  // namespace
 
 extern "C" int t0mi_f32_to_bf16(t0mi_ctx* ctx, uint64_t src_f32, uint64_t dst_bf16, uint64_t count) {
@@ -262,10 +274,11 @@ extern "C" int t0mi_matmul_f32(t0mi_ctx* ctx, uint64_t x, uint64_t w, uint64_t y
   if (rc) return rc;
   T0MI_SUBMIT_GUARD(ctx);
   if (m == 0 || n == 0) return T0MI_OK;
-  if ((rc = run_gemm_f32(ctx, F32_FORWARD, x, w, y, m, n, k)) <= 0) return rc;
   const uint32_t kp = up8(k), np = up8(n);
   const size_t xa = align256((size_t)m * kp * 2), wb = align256((size_t)kp * np * 2);
   const size_t pad = np != n ? (size_t)m * np * 4 : 0;
+  if ((rc = run_gemm_f32(ctx, F32_FORWARD, x, w, y, m, n, k)) < 0) return rc;
+  if (rc == T0MI_OK) return hold_passes(ctx, xa + wb + pad, T0MI_NN, m, np, kp);
   rc = ensure_cvt_buffer(ctx, xa + wb + pad);
   if (rc) return rc;
   if (ctx->null_backend) return T0MI_OK;
@@ -284,8 +297,10 @@ extern "C" int t0mi_matmul_wt_bf16(t0mi_ctx* ctx, uint64_t x, uint64_t wt_bf16, 
   if (k % 8 || n % 8) return set_error(T0MI_ERR_INVALID, "K=%u and N=%u must be multiples of 8 (WT is used in place)", k, n);
   if (wt_bf16 & 15) return set_error(T0MI_ERR_INVALID, "WT must be 16-byte aligned");
   if (m == 0 || n == 0) return T0MI_OK;
-  if ((rc = run_gemm_wt(ctx, x, wt_bf16, y, m, n, k)) <= 0) return rc;
-  rc = ensure_cvt_buffer(ctx, align256((size_t)m * k * 2));
+  const size_t xa = align256((size_t)m * k * 2);
+  if ((rc = run_gemm_wt(ctx, x, wt_bf16, y, m, n, k)) < 0) return rc;
+  if (rc == T0MI_OK) return hold_passes(ctx, xa, T0MI_NT, m, n, k);
+  rc = ensure_cvt_buffer(ctx, xa);
   if (rc) return rc;
   if (ctx->null_backend) return T0MI_OK;
   if ((rc = cvt(ctx, x, (uint16_t*)ctx->cvt, m, m, k, k))) return rc;
@@ -300,10 +315,11 @@ extern "C" int t0mi_matmul_backward_data(t0mi_ctx* ctx, uint64_t dy, uint64_t w,
   if (rc) return rc;
   T0MI_SUBMIT_GUARD(ctx);
   if (m == 0 || k == 0) return T0MI_OK;
-  if ((rc = run_gemm_f32(ctx, F32_DATA, dy, w, dx, m, k, n)) <= 0) return rc;
   const uint32_t cp = up8(n), op = up8(k);  // contraction n, output columns k
   const size_t da = align256((size_t)m * cp * 2), wb = align256((size_t)op * cp * 2);
   const size_t pad = op != k ? (size_t)m * op * 4 : 0;
+  if ((rc = run_gemm_f32(ctx, F32_DATA, dy, w, dx, m, k, n)) < 0) return rc;
+  if (rc == T0MI_OK) return hold_passes(ctx, da + wb + pad, T0MI_NT, m, op, cp);
   rc = ensure_cvt_buffer(ctx, da + wb + pad);
   if (rc) return rc;
   if (ctx->null_backend) return T0MI_OK;
@@ -321,10 +337,11 @@ extern "C" int t0mi_matmul_backward_weight(t0mi_ctx* ctx, uint64_t x, uint64_t d
   if (rc) return rc;
   T0MI_SUBMIT_GUARD(ctx);
   if (k == 0 || n == 0) return T0MI_OK;
-  if ((rc = run_gemm_f32(ctx, F32_WEIGHT, x, dy, dw, k, n, m)) <= 0) return rc;
   const uint32_t cp = up8(m), np = up8(n);  // contraction m, output columns n
   const size_t xa = align256((size_t)k * cp * 2), db = align256((size_t)cp * np * 2);
   const size_t pad = np != n ? (size_t)k * np * 4 : 0;
+  if ((rc = run_gemm_f32(ctx, F32_WEIGHT, x, dy, dw, k, n, m)) < 0) return rc;
+  if (rc == T0MI_OK) return hold_passes(ctx, xa + db + pad, T0MI_NN, k, np, cp);
   rc = ensure_cvt_buffer(ctx, xa + db + pad);
   if (rc) return rc;
   if (ctx->null_backend) return T0MI_OK;

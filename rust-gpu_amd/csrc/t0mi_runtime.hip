@@ -164,6 +164,10 @@ int ensure_cvt_buffer(t0mi_ctx* ctx, size_t bytes) {
   return grow(ctx, "the conversion buffer", &ctx->cvt, &ctx->cvt_bytes, bytes);
 }
 
+int try_cvt_buffer(t0mi_ctx* ctx, size_t bytes, bool* ok) {
+  return grow(ctx, "the conversion buffer", &ctx->cvt, &ctx->cvt_bytes, bytes, ok);
+}
+
 int xk_prepare(t0mi_ctx* ctx, uint32_t tiles, size_t part_bytes, XcdExchange* x, bool* ok, bool optional) {
   *ok = false;
   if (ctx->null_backend || ctx->xk_nx == 0) return T0MI_OK;
@@ -1164,6 +1168,18 @@ bool cached_auto_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t transpose, ui
 }
 }  // namespace
 
+bool t0mi::gemm_auto_workspace(t0mi_ctx* ctx, uint32_t transpose, uint32_t m, uint32_t n, uint32_t k,
+                               uint32_t out_dtype, size_t* bytes) {
+  *bytes = 0;
+  if (transpose == T0MI_NT && gemm_decode_nt_takes(ctx, m, n, k)) return true;
+  AutoPlan pl;
+  if (!cached_auto_plan(m, n, k, transpose, out_dtype, (uint32_t)ctx->cu_count, &pl)) return false;
+  const size_t sk_h = split_k_of(pl.head), sk_t = pl.n1 < n ? split_k_of(pl.tail) : 1;
+  if (sk_h > 1) *bytes = (size_t)m * pl.n1 * 4 * sk_h;
+  if (sk_t > 1) *bytes = std::max(*bytes, (size_t)m * (n - pl.n1) * 4 * sk_t);
+  return true;
+}
+
 int t0mi::run_gemm_auto(t0mi_ctx* ctx, uint32_t transpose, uint64_t x, uint64_t b, uint64_t y, uint32_t m, uint32_t n,
                         uint32_t k, uint32_t out_dtype, uint64_t bias, const EpiChain* epi) {
   if (transpose == T0MI_NT) {
@@ -1222,11 +1238,8 @@ static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm
                          const EpiChain& chain) {
   const bool valid = m && n && k && k % 8 == 0 && n % 8 == 0 && !((x | b | y) & 15) && !(bias & 3) &&
                      !(chain_uses(chain, EOP_BIAS) && !bias);
-  AutoPlan pl;
-  if (tile_split_k(s) == 1 && valid &&
-      cached_auto_plan(m, n, k, cfg.transpose, cfg.out_dtype, (uint32_t)ctx->cu_count, &pl)) {
-    const uint32_t sk_h = split_k_of(pl.head), sk_t = pl.n1 < n ? split_k_of(pl.tail) : 1;
-    const size_t need = std::max(sk_h > 1 ? (size_t)m * pl.n1 * 4 * sk_h : 0, sk_t > 1 ? (size_t)m * (n - pl.n1) * 4 * sk_t : 0);
+  size_t need = 0;
+  if (tile_split_k(s) == 1 && valid && gemm_auto_workspace(ctx, cfg.transpose, m, n, k, cfg.out_dtype, &need)) {
     bool ok = false;
     if (int rc = try_workspace(ctx, need, &ok)) return rc;
     if (ok) return run_gemm_auto(ctx, cfg.transpose, x, b, y, m, n, k, cfg.out_dtype, bias, &chain);

@@ -128,3 +128,24 @@ done([before, out])
     before, out = r
     assert all(c[1] is None and c[2] == before for c in out.values()), out
     assert out["f32"][0] == ["gemm_f32_kernel"] and out["tile"][0] == ["gemm_bf16_kernel"]
+
+
+@pytest.mark.parametrize("call,warm,then", [
+    ("lambda m: rt.matmul(X, B, Y, m, 4230, 522)", 1659, 1004),            # passes below the one launch
+    ("lambda m: rt.matmul_with_wt_bf16(X, B, Y, m, 4096, 4096)", 16, 1),   # the persistent decode
+    ("lambda m: rt.matmul_with_wt_bf16(X, B, Y, m, 4376, 2912)", 38, 37),  # the scheduled GEMM's planes
+    ("lambda m: rt.matmul_backward_data(X, B, Y, m, 688, 1529)", 1037, 933),
+    ("lambda k: rt.matmul_backward_weight(X, B, Y, 6350, k, 522)", 1257, 1052),  # the layer's width
+])
+def test_smaller_batches_captured_after_the_largest(host, call, warm, then):
+    """A call runs once at its largest batch, in one launch; at a smaller batch, captured, it takes the
+    conversion passes, whose buffers the first call made as well."""
+    r = host(f"""
+call = {call}
+a = names(call, {warm})
+rt.capture_begin()
+b = names(call, {then})
+rt.capture_end()
+done([a, b])
+""")
+    assert r[0][-1] == "gemm_f32_kernel" and r[1][0].startswith("cvt_bf16"), r
