@@ -960,13 +960,13 @@ extern "C" int t0mi_wait_idle(t0mi_ctx* ctx) {
 // ---------------------------------------------------------- one-call GEMM ----
 
 namespace t0mi {
-// Whether the bytes of Y[m,n] meet those of X, B or the bias (row length ld of Y and of NN's B).
-static bool output_meets_operands(const t0mi_gemm_config& cfg, uint64_t x, uint64_t b, uint64_t y, uint64_t bias,
-                                  uint32_t m, uint32_t n, uint32_t k, uint32_t ld) {
+// Whether the bytes of Y[m,n] meet those of X or B (row length ld of Y and of NN's B).  The bias is no
+// matter here: the reduce, too, reads it while it writes Y.
+static bool output_meets_operands(const t0mi_gemm_config& cfg, uint64_t x, uint64_t b, uint64_t y, uint32_t m,
+                                  uint32_t n, uint32_t k, uint32_t ld) {
   const uint64_t y_bytes = ((uint64_t)(m - 1) * ld + n) * (cfg.out_dtype == T0MI_OUT_BF16 ? 2 : 4);
   const uint64_t b_bytes = (cfg.transpose == T0MI_NN ? (uint64_t)(k - 1) * ld + n : (uint64_t)n * k) * 2;
-  return ranges_meet(x, (uint64_t)m * k * 2, y, y_bytes) || ranges_meet(b, b_bytes, y, y_bytes) ||
-         (bias && ranges_meet(bias, (uint64_t)n * 4, y, y_bytes));
+  return ranges_meet(x, (uint64_t)m * k * 2, y, y_bytes) || ranges_meet(b, b_bytes, y, y_bytes);
 }
 
 int run_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e, uint64_t x, uint64_t b,
@@ -1039,7 +1039,7 @@ int run_gemm(t0mi_ctx* ctx, const t0mi_gemm_config& cfg, const GemmLaunchEntry* 
   p.k_per_split = ((kt + sk - 1) / sk) * cfg.tile_k;
   const size_t slots = (size_t)p.tiles_m * p.tiles_n * sk * cfg.tile_m * cfg.tile_n * 4;
   if (e->fn_exchange && !fixed && sk == 2 && slots <= kExchangeSlotBytes &&
-      !output_meets_operands(cfg, x, b, y, bias, m, n, k, ld)) {
+      !output_meets_operands(cfg, x, b, y, m, n, k, ld)) {
     XcdExchange xk;
     bool ok = false;
     rc = xk_prepare(ctx, p.tiles_m * p.tiles_n, kExchangeSlotBytes, &xk, &ok, true);
