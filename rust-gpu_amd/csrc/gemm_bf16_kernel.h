@@ -876,7 +876,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_exchange_kernel(GemmPa
   gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, kSumsExchange>(p, tm, tn, part, &xk);
 }
 
-// Planes only, without the epilogue's code.
+// Split-K planes, without the epilogue's code.
 template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_planes_kernel(GemmParams p) {
   int tm, tn, part;

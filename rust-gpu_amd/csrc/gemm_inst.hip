@@ -23,9 +23,13 @@ static void launch_variant(dim3 g, hipStream_t s, const GemmParams& p) {
       return;
     }
   }
-  // Split-K of the tiles that the ranked schedule splits: a kernel without the epilogue's code
-  // (128x4096x4096, 64x128 in 4 parts: 14.0-14.3 us with it in the kernel, 13.9 without).
-  if constexpr (BM * BN <= 128 * 128 && BK == 64 && WM * WN == 4 && S >= 3) {
+  // Split-K's planes: a kernel without the epilogue's code, whose chain and biases take up to twice the
+  // registers of the rest (128x128x16 on two waves: 62 VGPRs and two waves a SIMD, 234 and one with it).
+  // 2048x4096x1024 NN in 2 parts, 128x128x16: 55.1 us with the code in the kernel, 44.2 without; 64x128x16
+  // 54.9 and 45.6; 1024x2048x2048 NT in 8 parts, 256x128x32: 40.3 and 36.0; 128x4096x4096 NN in 4, 64x128x64:
+  // 14.0-14.3 and 13.9.  Single waves of up to 64x64 keep the one kernel: with more of them on a SIMD they
+  // run 4-6 % slower (2048x4096x1024 in 2 parts, 32x64x16 NN 62.1 and 66.1 us, 64x64x16 NT 67.2 and 70.5).
+  if constexpr (WM * WN > 1 || BM * BN > 64 * 64) {
     if (p.split_k > 1) {
       hipLaunchKernelGGL((gemm_bf16_planes_kernel<BM, BN, BK, WM, WN, S, NN>), g, dim3(WM * WN * 64), 0, s, p);
       return;

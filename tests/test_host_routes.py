@@ -149,3 +149,27 @@ rt.capture_end()
 done([a, b])
 """)
     assert r[0][-1] == "gemm_f32_kernel" and r[1][0].startswith("cvt_bf16"), r
+
+
+def test_split_k_planes_run_the_kernel_without_the_epilogue(host):
+    """Every prebuilt tile but single waves of up to 64x64 writes its planes with gemm_bf16_planes_kernel (the
+    256x256 ping-pong kernel has its own); the chain then runs in the reduce."""
+    r = host("""
+import re
+out, buf = [], ctypes.create_string_buffer(1 << 16)
+t0mi.lib().t0mi_gemm_variants(buf, len(buf))
+for name in buf.value.decode().split(","):
+    v = [int(x) for x in re.findall("[0-9]+", name)] + [int(name.endswith("_nn"))]
+    cfg = t0mi.GemmConfig(tile_m=v[0], tile_n=v[1], tile_k=v[2], wave_m=v[3], wave_n=v[4], stages=v[5], transpose=v[6],
+                          wg_size=64 * v[3] * v[4], use_lds=1, double_buffer=1, n_col_passes=1, swap_grid=1, split_k=4,
+                          epilogue=t0mi.EPI_BIAS_ADD_RELU)
+    rt.gemm(cfg, X, B, Y, 256, 512, 2048, BIAS)
+    out.append([v, [l[0].split("<")[0] for l in launches() if "fill" not in l[0]]])
+done(out)
+""")
+    assert len(r) > 60
+    for (bm, bn, bk, wm, wn, st, nn), k in r:
+        pingpong = (bm, bn, bk, wm, wn, st) == (256, 256, 64, 2, 4, 2)
+        one = wm * wn == 1 and bm * bn <= 64 * 64
+        want = "gemm_bf16_pingpong_kernel" if pingpong else "gemm_bf16_kernel" if one else "gemm_bf16_planes_kernel"
+        assert k == [want, "t0mi_splitk_reduce"], (bm, bn, bk, wm, wn, st, nn)
