@@ -1142,31 +1142,50 @@ namespace {
 // cached_auto_select's cache; cleared when it grows past kPlanCacheMax.
 struct PlanKey {
   uint32_t m, n, k, transpose, out_dtype, cus;
-  bool operator<(const PlanKey& o) const {
-    return std::tie(m, n, k, transpose, out_dtype, cus) < std::tie(o.m, o.n, o.k, o.transpose, o.out_dtype, o.cus);
-  }
+  auto fields() const { return std::tie(m, n, k, transpose, out_dtype, cus); }
+  bool operator<(const PlanKey& o) const { return fields() < o.fields(); }
+  bool operator==(const PlanKey& o) const { return fields() == o.fields(); }
 };
 constexpr size_t kPlanCacheMax = 4096;
 std::mutex g_plan_mu;
 std::map<PlanKey, AutoPlan> g_plans;
 bool cached_auto_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t transpose, uint32_t out_dtype, uint32_t cus,
                       AutoPlan* pl) {
+  // This thread's last plan ahead of the map: a program often repeats a shape, and a call may ask twice
+  // (64x64x64, a TileGemm call of 3.6 us: two lookups in a map of some hundred shapes cost 0.4 us).
+  thread_local PlanKey last_key{};
+  thread_local AutoPlan last;
   const PlanKey key{m, n, k, transpose, out_dtype, cus};
+  if (m && key == last_key) {
+    *pl = last;
+    return true;
+  }
+  bool known = false;
   {
     std::lock_guard<std::mutex> lk(g_plan_mu);
     auto it = g_plans.find(key);
     if (it != g_plans.end()) {
       *pl = it->second;
-      return true;
+      known = true;
     }
   }
-  if (!t0mi::auto_plan(m, n, k, transpose, out_dtype, cus, pl)) return false;
-  std::lock_guard<std::mutex> lk(g_plan_mu);
-  if (g_plans.size() >= kPlanCacheMax) g_plans.clear();
-  g_plans[key] = *pl;
+  if (!known) {
+    if (!t0mi::auto_plan(m, n, k, transpose, out_dtype, cus, pl)) return false;
+    std::lock_guard<std::mutex> lk(g_plan_mu);
+    if (g_plans.size() >= kPlanCacheMax) g_plans.clear();
+    g_plans[key] = *pl;
+  }
+  last_key = key;
+  last = *pl;
   return true;
 }
 }  // namespace
+
+// Bytes of ctx->ws that a plan's partial planes need.
+static size_t plan_workspace(const AutoPlan& pl, uint32_t m, uint32_t n) {
+  const size_t sk_h = split_k_of(pl.head), sk_t = pl.n1 < n ? split_k_of(pl.tail) : 1;
+  return std::max(sk_h > 1 ? (size_t)m * pl.n1 * 4 * sk_h : 0, sk_t > 1 ? (size_t)m * (n - pl.n1) * 4 * sk_t : 0);
+}
 
 bool t0mi::gemm_auto_workspace(t0mi_ctx* ctx, uint32_t transpose, uint32_t m, uint32_t n, uint32_t k,
                                uint32_t out_dtype, size_t* bytes) {
@@ -1174,9 +1193,7 @@ bool t0mi::gemm_auto_workspace(t0mi_ctx* ctx, uint32_t transpose, uint32_t m, ui
   if (transpose == T0MI_NT && gemm_decode_nt_takes(ctx, m, n, k)) return true;
   AutoPlan pl;
   if (!cached_auto_plan(m, n, k, transpose, out_dtype, (uint32_t)ctx->cu_count, &pl)) return false;
-  const size_t sk_h = split_k_of(pl.head), sk_t = pl.n1 < n ? split_k_of(pl.tail) : 1;
-  if (sk_h > 1) *bytes = (size_t)m * pl.n1 * 4 * sk_h;
-  if (sk_t > 1) *bytes = std::max(*bytes, (size_t)m * (n - pl.n1) * 4 * sk_t);
+  *bytes = plan_workspace(pl, m, n);
   return true;
 }
 
@@ -1238,11 +1255,17 @@ static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm
                          const EpiChain& chain) {
   const bool valid = m && n && k && k % 8 == 0 && n % 8 == 0 && !((x | b | y) & 15) && !(bias & 3) &&
                      !(chain_uses(chain, EOP_BIAS) && !bias);
-  size_t need = 0;
-  if (tile_split_k(s) == 1 && valid && gemm_auto_workspace(ctx, cfg.transpose, m, n, k, cfg.out_dtype, &need)) {
-    bool ok = false;
-    if (int rc = try_workspace(ctx, need, &ok)) return rc;
-    if (ok) return run_gemm_auto(ctx, cfg.transpose, x, b, y, m, n, k, cfg.out_dtype, bias, &chain);
+  if (tile_split_k(s) == 1 && valid) {
+    if (cfg.transpose == T0MI_NT) {
+      const int rc = run_gemm_decode_nt(ctx, x, b, y, m, n, k, cfg.out_dtype, bias, chain);
+      if (rc <= 0) return rc;
+    }
+    AutoPlan pl;
+    if (cached_auto_plan(m, n, k, cfg.transpose, cfg.out_dtype, (uint32_t)ctx->cu_count, &pl)) {
+      bool ok = false;
+      if (int rc = try_workspace(ctx, plan_workspace(pl, m, n), &ok)) return rc;
+      if (ok) return run_gemm_planned(ctx, pl, cfg.transpose, x, b, y, m, n, k, cfg.out_dtype, bias, &chain);
+    }
   }
   return run_gemm(ctx, cfg, e, x, b, y, bias, m, n, k, chain);
 }
