@@ -1247,15 +1247,16 @@ extern "C" int t0mi_auto_gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t 
 // open, and its tile is one of an RDNA part's (64 x 64 x 16 on one wave, say), so the schedule that
 // auto_select ranks first for the shape runs under the spec's name, kernargs and grid, as for the
 // persistent presets (1000 x 2752 x 2056 NT, bias + GELU, bf16 out, tile_auto_select's 64x64 k16: 63.8
-// us on its own tile, 24.1 so).  The spec's tile remains for specs that name their split-K, for
-// calls whose arguments are refused (it reports them), and where the schedule's split-K planes would
+// us on its own tile, 24.1 so).  The spec's tile remains for specs that name their split-K, where Y
+// lies over X or B (one tile, the whole of Y, is stored after its operands are read; the schedule may
+// cut it into several), for calls whose arguments are refused (it reports them), and where the schedule's split-K planes would
 // need workspace that cannot be had now (a capture, live graphs holding its address, no memory left).
 static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e,
                          uint64_t x, uint64_t b, uint64_t y, uint64_t bias, uint32_t m, uint32_t n, uint32_t k,
                          const EpiChain& chain) {
   const bool valid = m && n && k && k % 8 == 0 && n % 8 == 0 && !((x | b | y) & 15) && !(bias & 3) &&
                      !(chain_uses(chain, EOP_BIAS) && !bias);
-  if (tile_split_k(s) == 1 && valid) {
+  if (tile_split_k(s) == 1 && valid && !output_meets_operands(cfg, x, b, y, m, n, k, n)) {
     if (cfg.transpose == T0MI_NT) {
       const int rc = run_gemm_decode_nt(ctx, x, b, y, m, n, k, cfg.out_dtype, bias, chain);
       if (rc <= 0) return rc;

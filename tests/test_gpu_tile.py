@@ -57,6 +57,21 @@ def test_presets_integer_exact(rt, preset, nn):
     assert np.array_equal(y, ref), preset
 
 
+@pytest.mark.parametrize("nn", [0, 1])
+def test_output_over_an_operand(rt, nn):
+    """Y in X's or B's place, all of it one tile of the spec: stored after its operands are read."""
+    m = n = k = 128
+    spec = t0mi.tile_preset("tile_128x128_k32").copy(transpose=nn, out_dtype=t0mi.OUT_BF16)
+    a, b = oracle.normal_bf16((m, k), 31, 0.0, 1.0), oracle.normal_bf16((k, n), 32, 0.0, 1.0)
+    ref = oracle.gemm_bf16(a, b, "nn" if nn else "nt")
+    tol = oracle.gemm_tolerance(k, oracle.bf16_to_f32(a), oracle.bf16_to_f32(b))
+    for over in (0, 1):
+        dev = [to_dev(a), to_dev(b)]
+        rt.tile_gemm(spec, dev[0][1], dev[1][1], dev[over][1], m, n, k)
+        y = oracle.bf16_to_f32(from_dev(dev[over][0], np.uint16, (m, n)))
+        assert np.all(np.abs(y - ref) <= np.abs(ref) * 2.0 ** -8 + tol)
+
+
 OPS = [("bias", [t0mi.BIAS_ADD]), ("scale", [t0mi.SCALE]), ("relu", [t0mi.RELU]), ("silu", [t0mi.SILU]),
        ("gelu", [t0mi.GELU]), ("abs", [t0mi.ABS]), ("neg", [t0mi.NEG]), ("clamp", [t0mi.CLAMP]),
        ("bias_relu", [t0mi.BIAS_ADD, t0mi.RELU]),

@@ -173,3 +173,21 @@ done(out)
         one = wm * wn == 1 and bm * bn <= 64 * 64
         want = "gemm_bf16_pingpong_kernel" if pingpong else "gemm_bf16_kernel" if one else "gemm_bf16_planes_kernel"
         assert k == [want, "t0mi_splitk_reduce"], (bm, bn, bk, wm, wn, st, nn)
+
+
+@pytest.mark.parametrize("layout", ["NT", "NN"])
+def test_tile_spec_writes_y_after_the_operands_are_read(host, layout):
+    """Y over X or B, all of it inside the spec's one tile: that tile's kernel, which stores Y after its
+    last read; the ranked schedule would cut it into several."""
+    r = host(f"""
+spec = t0mi.tile_preset("tile_128x128_k32").copy(transpose=t0mi.{layout}, out_dtype=t0mi.OUT_BF16)
+def run(y):
+    rt.tile_gemm(spec, X, B, y, 128, 128, 128)
+    return [l[0] + " %d" % (l[1] * l[2]) for l in launches()]
+rt.tile_gemm(spec, X, B, Y, 128, 128, 128)
+hip.fake_launches()
+done([run(Y), run(X), run(B), run(X + 128 * 128 * 2 - 16), run(X + 128 * 128 * 2)])
+""")
+    own = f"gemm_bf16_kernel<128,128,32,2,2,2,{str(layout == 'NN').lower()}> 1"
+    assert r[0] == r[4] != [own]
+    assert r[1] == r[2] == r[3] == [own]
