@@ -694,8 +694,15 @@ extern "C" int t0mi_w4a16_gemm(t0mi_ctx* ctx, uint64_t a, uint64_t qweight, uint
   // launch (one pass over the weights feeds them all), spread evenly over the
   // fewest launches (5 slabs as 3 + 2, not 4 + 1); the other kernels one.
   const uint32_t slabs = (m + 15) / 16;
-  // Planes of every row (several tiles in one launch) only where the workspace can hold them now.
+  // Planes of every row (several tiles in one launch) only where the workspace can hold them now; and one
+  // tile at a time where Y lies over an operand, which a single strip reads before it stores.
   uint32_t tile_rs = v2 ? decode_row_tiles(slabs, decode_max_slabs(group), strips * ky, (uint32_t)ctx->cu_count) : 0;
+  const uint64_t y_bytes = (uint64_t)m * n * (p.out_bf16 ? 2 : 4), params = (uint64_t)(k / group) * n;
+  if (tile_rs && (ranges_meet(a, (uint64_t)m * k * 2, y, y_bytes) ||
+                  ranges_meet(qweight, (uint64_t)k * n / 2, y, y_bytes) ||
+                  ranges_meet(scales, params * 2, y, y_bytes) ||
+                  (qzeros && ranges_meet(qzeros, params / 2, y, y_bytes))))
+    tile_rs = 0;
   if (tile_rs && ky > 1) {
     bool ok = false;
     rc = try_workspace(ctx, (size_t)m * n * 4 * ky, &ok);

@@ -57,3 +57,17 @@ def test_row_tiles(rt, m, k, n, group, zeros):
     for r0, rows in ((0, min(m, 48)), (16, m - 16)):  # other tilings of the same rows, over 16 rows each
         if rows > 16:
             assert np.array_equal(call(r0, rows), y[r0:r0 + rows]), (r0, rows)
+
+
+def test_output_over_the_activations(rt):
+    """One strip and one launch of four slabs: Y (f32, the size of A) in A's place."""
+    m, k, n, group = 64, 128, 64, 128
+    a = oracle.normal_bf16((m, k), 5, 0.0, 1.0)
+    w = oracle.pack_qweight(oracle.nibbles((k, n), 6))
+    s = oracle.uniform_bf16((k // group, n), 7, 0.005, 0.02)
+    (da, pa), (dw, pw), (ds, ps) = to_dev(a), to_dev(w), to_dev(s)
+    dy, py = empty_dev(m * n * 4, fill=0xCD)
+    rt.w4a16_gemm(pa, pw, ps, 0, 8, py, m, k, n, group, t0mi.OUT_F32)
+    want = from_dev(dy, np.float32, (m, n))
+    rt.w4a16_gemm(pa, pw, ps, 0, 8, pa, m, k, n, group, t0mi.OUT_F32)
+    assert np.array_equal(from_dev(da, np.float32, (m, n)), want)

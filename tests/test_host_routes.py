@@ -191,3 +191,20 @@ done([run(Y), run(X), run(B), run(X + 128 * 128 * 2 - 16), run(X + 128 * 128 * 2
     own = f"gemm_bf16_kernel<128,128,32,2,2,2,{str(layout == 'NN').lower()}> 1"
     assert r[0] == r[4] != [own]
     assert r[1] == r[2] == r[3] == [own]
+
+
+def test_w4a16_row_tiles_apart_from_the_operands(host):
+    """A weight of one 64-column strip, up to 64 rows: one workgroup reads everything and then stores Y, which
+    may lie over an operand; side by side, one row tile's Y would lie over another's activations."""
+    r = host("""
+m, k, n, group = 64, 128, 64, 128  # four slabs in one launch
+S, Z = 5 << 40, 6 << 40
+def grid(y, z=Z):
+    rt.w4a16_gemm(X, B, S, z, 8, y, m, k, n, group, t0mi.OUT_F32)
+    return launches()[-1][1:4]
+grid(Y)
+done(dict(apart=[grid(Y), grid(X + m * k * 2), grid(Y, 0)],
+          over=[grid(y) for y in (X, X + m * k * 2 - 16, B, S, Z)]))
+""")
+    assert r["apart"] == [[1, 1, 4]] * 3
+    assert r["over"] == [[1, 1, 1]] * 5
