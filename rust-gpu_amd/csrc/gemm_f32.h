@@ -222,16 +222,14 @@ __global__ __launch_bounds__(WM* WN* G * 64) void gemm_f32_kernel(GemmF32Params 
 
   // Workgroup -> (tile, K piece).  Neighbouring tiles share an XCD (and its L2).
   int tm, tn, part;
-  uint32_t tile = 0, piece = 0;
+  uint32_t tile = 0, piece = 0, counter = 0;
   if (p.pieces == 1) {
     tile_coords_of(p.tiles_m, p.tiles_n, 1, tm, tn, part);
   } else {
     xk_check_placement(p.x);
-    xk_unpack(blockIdx.x, p.x.nx, p.pieces, &tile, &piece);
-    const uint32_t tiles = p.tiles_m * p.tiles_n, per = (tiles + p.x.nx - 1) / p.x.nx;
-    const uint32_t idx = (tile % p.x.nx) * per + tile / p.x.nx;
-    if (idx >= tiles) return;
-    tile_coords_lin(idx, tiles, p.tiles_m, p.tiles_n, 0, tm, tn, part);
+    const uint32_t tiles = p.tiles_m * p.tiles_n;
+    if (!f32_workgroup(blockIdx.x, p.x.nx, p.pieces, tiles, &tile, &piece, &counter)) return;
+    tile_coords_lin(tile, tiles, p.tiles_m, p.tiles_n, 0, tm, tn, part);
   }
   const int M = (int)p.M, N = (int)p.N;
   const int nkt = ((int)p.K + BK - 1) / BK;  // K tiles, cut evenly over the pieces
@@ -366,7 +364,7 @@ __global__ __launch_bounds__(WM* WN* G * 64) void gemm_f32_kernel(GemmF32Params 
 #pragma unroll
     for (int j = 0; j < NOUT; ++j)
       if (act) xk_store(sl, piece * SLOT + o + (uint32_t)(j * ROWS_PER * BN * 4), __builtin_bit_cast(xk_f32x4, s[j]));
-    if (!xk_arrive(p.x, tile, p.pieces)) return;
+    if (!xk_arrive(p.x, counter, p.pieces)) return;
 #pragma unroll
     for (int j = 0; j < NOUT; ++j) s[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     for (uint32_t q0 = 0; q0 < p.pieces; q0 += 2) {  // pieces are a power of two
@@ -380,7 +378,7 @@ __global__ __launch_bounds__(WM* WN* G * 64) void gemm_f32_kernel(GemmF32Params 
 #pragma unroll
       for (int j = 0; j < NOUT; ++j) s[j] = s[j] + u[0][j] + u[1][j];
     }
-    xk_reset(p.x, tile);
+    xk_reset(p.x, counter);
   }
   const bool whole = n0 == ns && n0 + BN <= N;  // every column is this tile's and inside N
 #pragma unroll

@@ -73,6 +73,16 @@ T0MI_HD constexpr uint32_t f32_piece_off(bool kmajor, uint32_t ld, int first, in
   if (kmajor) return ((uint32_t)r * ld + (uint32_t)(first + sp * 4)) * 4u;
   return first + r < rows ? ((uint32_t)(first + r) * ld + (uint32_t)(sp * 4)) * 4u : kF32Oob;
 }
+// Workgroup `b` of a launch that cuts K over `pieces` workgroups a tile: the tile (its slots, and the order
+// in which neighbours share an XCD), the K piece and the number whose counter the tile's pieces share.  False:
+// the numbering's padding.  The numbers go past the tiles where these are no multiple of the XCDs; the
+// slots do not.
+T0MI_HD bool f32_workgroup(uint32_t b, uint32_t nx, uint32_t pieces, uint32_t tiles, uint32_t* tile,
+                           uint32_t* piece, uint32_t* counter) {
+  xk_unpack(b, nx, pieces, counter, piece);
+  *tile = *counter % nx * ((tiles + nx - 1) / nx) + *counter / nx;
+  return *tile < tiles;
+}
 // First K tile of piece q of p over nkt K tiles (piece q ends where q + 1 starts).
 T0MI_HD constexpr int f32_piece_begin(int q, int p, int nkt) { return (int)((int64_t)q * nkt / p); }
 

@@ -73,6 +73,28 @@ static void cover(const F32Plan& p, const F32Tiles& t, int mode, unsigned m, uns
   }
 }
 
+// A launch that cuts K: every (tile, piece) once, slots within the tiles' own, counters apart and within
+// an XCD's share.
+static void workgroups(const F32Plan& p, int mode, unsigned m, unsigned n, unsigned k) {
+  if (p.pieces == 1) return;
+  const uint32_t nx = 8, tiles = p.tiles_m * p.tiles_n, grid = (tiles + nx - 1) / nx * nx * p.pieces;
+  std::vector<int> hit(tiles * p.pieces, 0), at(tiles, -1);
+  bool ok = true;
+  for (uint32_t b = 0; b < grid; ++b) {
+    uint32_t tile, piece, counter;
+    if (!f32_workgroup(b, nx, p.pieces, tiles, &tile, &piece, &counter)) continue;
+    ok = ok && tile < tiles && piece < p.pieces && counter / nx < (tiles + nx - 1) / nx;
+    if (!ok) break;
+    ++hit[tile * p.pieces + piece];
+    ok = at[tile] < 0 || at[tile] == (int)counter;
+    at[tile] = (int)counter;
+  }
+  for (int h : hit) ok = ok && h == 1;
+  for (uint32_t i = 0; i < tiles && ok; ++i)
+    for (uint32_t j = 0; j < i; ++j) ok = ok && at[i] != at[j];
+  check(ok, "workgroups", mode, m, n, k);
+}
+
 // The bf16 weight's route: n and k multiples of 8 (what the entry point takes), up to 64 rows.
 static void wt(unsigned m, unsigned n, unsigned k, int split, int* used) {
   const F32Plan p = wt_plan(m, n, k, 256, split);
@@ -81,6 +103,7 @@ static void wt(unsigned m, unsigned n, unsigned k, int split, int* used) {
   const F32Tiles& t = kWtTiles[p.tile];
   check(m <= kWtMaxRows && (split || p.pieces == 1), "wt range", 3, m, n, k);
   cover(p, t, 3, m, n, k);
+  workgroups(p, 3, m, n, k);
   const uint64_t bytes = (uint64_t)n * k * 2;
   for (int tn : {0, (int)p.tiles_n - 1})
     for (int kt : {0, ((int)k - 1) / kF32Bk})
@@ -105,6 +128,7 @@ static void one(int mode, unsigned m, unsigned n, unsigned k, int split, std::ve
   ++used[p.tile * 4 + lp];
   check(split || p.pieces == 1, "pieces without the exchange", mode, m, n, k);
   cover(p, t, mode, m, n, k);
+  workgroups(p, mode, m, n, k);
   const int nkt = ((int)k + kF32Bk - 1) / kF32Bk;
   // Loads: first, second last and last tile of each dimension, first and last K tiles.
   for (int kt : {0, nkt / 2, nkt - 1})
