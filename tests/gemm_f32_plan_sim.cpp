@@ -141,7 +141,22 @@ static void one(int mode, unsigned m, unsigned n, unsigned k, int split, std::ve
     }
 }
 
+// Calls near the line whose measured times are more than 1.15 apart: the faster route.
+static void routes() {
+  const struct {
+    int mode;
+    unsigned m, n, k;
+    bool one_launch;
+  } c[] = {{F32_DATA, 696, 192, 8128, false},   {F32_DATA, 564, 344, 7232, false},  {F32_FORWARD, 927, 320, 7232, false},
+           {F32_DATA, 653, 384, 7424, false},   {F32_FORWARD, 886, 216, 7408, false}, {F32_FORWARD, 622, 328, 7984, false},
+           {F32_DATA, 91, 1280, 6784, true},    {F32_FORWARD, 79, 1408, 4544, true}, {F32_DATA, 222, 2048, 6912, true},
+           {F32_FORWARD, 69, 3800, 5672, true}, {F32_FORWARD, 436, 417, 6683, true}};
+  for (const auto& x : c)
+    check((f32_plan(x.mode, x.m, x.n, x.k, 256, true).tile >= 0) == x.one_launch, "route", x.mode, x.m, x.n, x.k);
+}
+
 int main() {
+  routes();
   std::vector<int> used(kF32TileCount * 4 + 1, 0);
   srand(1);
   const unsigned edge[] = {1, 2, 3, 4, 5, 7, 8, 15, 16, 31, 32, 33, 63, 64, 65, 66, 100, 127, 128, 129, 255, 333, 1000, 4096};
