@@ -100,14 +100,21 @@ def test_f32_product(rt, mode, m, n, k):
         assert th.equal(y, z), "a second call differs"
 
 
-@pytest.mark.parametrize("m,n,k", [
+# (m, n, k), on the 32x64 tile but for the last three
+WT_SHAPES = [
     (1, 8, 8), (3, 200, 40),   # one cut K tile, columns short of the tile
-    (7, 11008, 2048),          # 32x64
-    (17, 520, 3000),           # 32x64, K pieces, K % 32 != 0
+    (7, 11008, 2048),
+    (17, 520, 3000),           # K pieces, K % 32 != 0
     (16, 512, 8192),           # 8 pieces
-    (33, 1000, 264), (64, 4096, 1032),  # two row tiles / 64x64
+    (33, 1000, 264), (64, 4096, 1032),  # two row tiles
     (64, 72, 4096),
-])
+    (44, 9960, 264),           # 64x64, K % 32 != 0
+    (64, 13000, 72),           # 64x64, three K tiles, the last one cut
+    (62, 3672, 7288),          # 64x64, 4 pieces, K % 32 != 0
+]
+
+
+@pytest.mark.parametrize("m,n,k", WT_SHAPES)
 def test_bf16_weight(rt, m, n, k):
     """matmul_with_wt_bf16 (bf16_matmul.rs:99-134): X f32, WT bf16 in place; same bars."""
     th = torch()

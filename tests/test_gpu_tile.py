@@ -12,7 +12,7 @@ import pytest
 
 import oracle
 import t0mi
-from gpu_helpers import empty_dev, from_dev, runtime, to_dev
+from gpu_helpers import empty_dev, from_dev, runtime, to_dev, torch
 
 pytestmark = pytest.mark.gpu
 
@@ -48,13 +48,49 @@ def run_tile(rt, spec, a, b, m, n, k, bias=None, scale=1.0, lo=0.0, hi=0.0):
 @pytest.mark.parametrize("preset", PRESETS)
 @pytest.mark.parametrize("nn", [0, 1])
 def test_presets_integer_exact(rt, preset, nn):
-    # NN tiles narrower than 64 columns run on the 64-column NN kernel; tile_k 48 as three 16-K steps.
+    # One-shot specs run the ranked schedule here; test_presets_own_tile runs their own kernels.
     spec = t0mi.tile_preset(preset).copy(transpose=nn)
     m, n, k = 200, 136, 264
     a, b = int_pattern(m, k, n, nn)
     y = run_tile(rt, spec, a, b, m, n, k)
     ref = oracle.gemm_bf16(a, b, "nn" if nn else "nt")
     assert np.array_equal(y, ref), preset
+
+
+@pytest.mark.parametrize("preset", [p for p in PRESETS if "persistent" not in p])
+@pytest.mark.parametrize("nn", [0, 1])
+def test_presets_own_tile(preset, nn):
+    """The spec's own kernel, which runs where the ranked schedule's planes cannot be held: captured on a
+    runtime without workspace, a shape whose schedule splits K.  NN tiles narrower than 64 columns run on
+    the 64-column NN kernel; tile_k 48 as three 16-K steps."""
+    th = torch()
+    m, n, k = 128, 1032, 1032
+    ops = [t0mi.BIAS_ADD, t0mi.RELU]
+    spec = t0mi.tile_preset(preset).copy(transpose=nn, epilogue=ops)
+    a, b = int_pattern(m, k, n, nn)
+    bias = ((np.arange(n) % 9) - 4).astype(np.float32)
+    ref = oracle.epilogue(oracle.gemm_bf16(a, b, "nn" if nn else "nt"), ops, bias=bias)
+    st = th.cuda.Stream()
+    with th.cuda.stream(st):
+        r = t0mi.Runtime(device=0, stream=st.cuda_stream)
+        (da, pa), (db, pb), (dc, pc) = to_dev(a), to_dev(b), to_dev(bias)
+        dy, py = empty_dev(m * n * 4, fill=0xAB)
+        st.synchronize()
+        g = None
+        try:
+            r.capture_begin()
+            r.tile_gemm(spec, pa, pb, py, m, n, k, bias=pc)
+            g = r.capture_end()
+            assert g.node_count == 1  # no reduce
+            for _ in range(2):
+                dy[:m * n * 4].fill_(0xAB)
+                g.launch()
+                st.synchronize()
+                assert np.array_equal(from_dev(dy, np.float32, (m, n)), ref), preset
+        finally:  # before the stream and the HIP runtime go
+            if g:
+                g.destroy()
+            r.close()
 
 
 @pytest.mark.parametrize("nn", [0, 1])

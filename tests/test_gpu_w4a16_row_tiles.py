@@ -4,7 +4,7 @@ slabs side by side.  Every row goes through the operations of a 16-row slab what
 f32 results equal, bit for bit, those of the same rows inside a call that tiles them differently; and
 they are within the fp32 bound k * 2^-24 * sum |a w| (times 2) of the exact product.
 Cases: a last tile of one row, of one slab, tiles of 1, 2, 3 and 4 slabs, planes over K (K > 4096) with
-tiles, groups 32 to 256, widths off the strip."""
+tiles of one slab and of three, groups 32 to 256, widths off the strip (test_host_routes.py holds them to it)."""
 import numpy as np
 import pytest
 
@@ -22,16 +22,24 @@ def rt():
     r.close()
 
 
-@pytest.mark.parametrize("m,k,n,group,zeros", [
+CASES = [
     (17, 1024, 520, 128, True),     # two tiles of one slab, the last one row
-    (33, 512, 4096, 64, False),     # three slabs
-    (100, 4096, 1376, 128, True),
-    (129, 512, 1000, 32, True),     # one row past eight slabs
-    (191, 1024, 4096, 128, False),  # four tiles of three slabs
-    (96, 2048, 520, 256, True),     # group 256: at most two slabs a tile
-    (112, 8192, 520, 128, True),    # planes over K and row tiles
-    (150, 512, 6000, 128, False),   # 94 strips
-])
+    (33, 512, 4096, 64, False),     # three of one
+    (100, 4096, 1376, 128, True),   # seven of one
+    (129, 512, 1000, 32, True),     # nine of one, one row past eight slabs
+    (191, 1024, 4096, 128, False),  # four of three
+    (96, 2048, 520, 256, True),     # group 256: six of one
+    (112, 8192, 520, 128, True),    # seven of one, planes over K
+    (150, 512, 6000, 128, False),   # five of two, 94 strips
+    (128, 512, 6000, 128, True),    # two of four
+    (100, 1024, 4096, 64, True),    # group 64: four of two
+    (112, 512, 5000, 32, False),    # group 32: three of three, the last one slab
+    (96, 512, 6000, 256, True),     # group 256: three of two
+    (185, 8192, 2048, 128, False),  # four of three, planes over K
+]
+
+
+@pytest.mark.parametrize("m,k,n,group,zeros", CASES)
 def test_row_tiles(rt, m, k, n, group, zeros):
     a = oracle.normal_bf16((m, k), 3 * m + n, 0.0, 1.0)
     w = oracle.pack_qweight(oracle.nibbles((k, n), m + 1))

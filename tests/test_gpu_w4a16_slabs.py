@@ -1,7 +1,9 @@
 """GPU parity of the multi-slab W4A16 decode launch (csrc/w4a16_decode.h, RS = 2
 to 4): for groups 32..256 t0mi_w4a16_gemm runs the decode kernel over up to four
-16-row slabs per launch (group 128; three for groups 32 and 64, two for 256) in
-one pass over the weights, spread evenly over the fewest launches.  Every row goes through the
+16-row slabs per workgroup (group 128; three for groups 32 and 64, two for 256) in
+one pass over the weights: on a wide weight one launch after another, spread evenly over
+the fewest, on a narrow one as row tiles side by side in one launch (CASES say which;
+test_host_routes.py holds them to it).  Every row goes through the
 operations of a 16-row launch of its own slab, so the result must be
 bit-identical to calling t0mi_w4a16_gemm on each 16-row slab separately where that call
 takes the one-slab kernel with one workgroup per 64-column strip (N > 8192 columns, or a
@@ -11,7 +13,7 @@ within the fp32 reordering bound 2 * K * 2^-24 * sum|a*w| (plus one bf16 ulp for
 and within the GEMM tolerance of the oracle (w = (q - z) * s, quant_kernels.rs:24, 95-100).
 Cases: 17..191 rows (odd remainders, a trailing one- or two-slab launch), groups
 32..256 (256: two chunks per wave, at most two slabs), per-group and constant zero points, f32 and bf16
-output, K beyond one workgroup's range (split-K planes of 64 rows + reduce),
+output, K beyond one workgroup's range (split-K planes + reduce),
 and the full decode width N = 11008.
 """
 import numpy as np
@@ -48,18 +50,27 @@ def call(rt, pa, pw, ps, pz, zp, m, k, n, group, out_bf16):
 
 CASES = [
     # (m, k, n, group, zeros, out_bf16)
+    # Narrow weights: row tiles of one slab.
     (17, 512, 200, 128, True, True),
     (31, 1024, 520, 64, False, True),
-    (32, 4096, 11008, 128, False, True),   # the decode shape with 32 rows
-    (33, 256, 136, 32, True, False),       # three slabs, the last one row
-    (48, 2048, 1000, 256, True, True),     # group 256: two chunks per wave, two slabs then one
-    (64, 8192, 256, 128, False, False),    # K split across workgroups: one four-slab launch, 64-row planes + reduce
-    (80, 384, 200, 128, True, True),       # three slabs, then two
-    (47, 512, 64, 64, False, True),
-    (48, 4096, 2048, 64, True, True),      # three slabs, 8-wave workgroups, no K split
-    (96, 4096, 520, 32, False, False),     # two three-slab launches, group 32
-    (112, 1024, 520, 128, True, True),     # group 128: four slabs, then three
-    (191, 4096, 1000, 128, False, True),   # group 128: three four-slab launches, the last 15 rows
+    (33, 256, 136, 32, True, False),       # the last one row
+    (48, 2048, 1000, 256, True, True),     # group 256: two chunks per wave
+    (64, 8192, 256, 128, False, False),    # K split across workgroups: 64-row planes + reduce
+    (80, 384, 200, 128, True, True),
+    (47, 512, 64, 64, False, True),        # one strip
+    (48, 4096, 2048, 64, True, True),      # 8-wave workgroups, no K split
+    (96, 4096, 520, 32, False, False),
+    (112, 1024, 520, 128, True, True),
+    (191, 4096, 1000, 128, False, True),   # twelve tiles, the last 15 rows
+    # Wide weights: several slabs in one launch after another.
+    (32, 4096, 11008, 128, False, True),   # the decode shape with 32 rows: two slabs
+    (48, 4096, 11008, 128, True, False),   # three
+    (100, 4096, 11008, 128, True, True),   # four, then three (the last four rows)
+    (64, 512, 16384, 128, False, True),    # four, 4-wave workgroups
+    (63, 4224, 11008, 128, True, True),    # K split across workgroups: planes of four slabs
+    (48, 512, 16384, 32, True, True),      # group 32: three
+    (90, 512, 11008, 64, False, False),    # group 64: three, then three
+    (70, 512, 11008, 256, True, True),     # group 256: two, two, one
 ]
 
 

@@ -1,8 +1,14 @@
 """Which kernels libt0mi launches for a call, and that a call which returned no error launched what it
 needs: the host side alone, with a stand-in for the HIP runtime (host_runtime.py).  The kernels'
-results are the GPU tests' matter."""
+results are the GPU tests' matter; the last tests here hold the cases of those to the kernels that they
+name."""
+import re
+
 import pytest
 
+import test_gpu_f32_gemm
+import test_gpu_w4a16_row_tiles
+import test_gpu_w4a16_slabs
 from host_runtime import host  # noqa: F401
 
 PLANES = ["gemm_bf16_planes_kernel", "t0mi_splitk_reduce"]
@@ -208,3 +214,75 @@ done(dict(apart=[grid(Y), grid(X + m * k * 2), grid(Y, 0)],
 """)
     assert r["apart"] == [[1, 1, 4]] * 3
     assert r["over"] == [[1, 1, 1]] * 5
+
+
+def test_every_preset_has_its_own_tile_under_capture(host):
+    r = host("""
+out = []
+for p in t0mi.tile_preset_names():
+    for nn in range(2):
+        spec = t0mi.tile_preset(p).copy(transpose=nn)
+        if spec.persistent:
+            continue
+        rt.capture_begin()
+        rt.tile_gemm(spec, X, B, Y, 128, 1032, 1032)
+        rt.capture_end()
+        out.append([[spec.tile_m, spec.tile_n, spec.tile_k, nn], [l[0] for l in launches()]])
+done(out)
+""")
+    assert len(r) == 46
+    for (m, n, k, nn), names in r:
+        bk = 64 if k % 64 == 0 else 32 if k % 32 == 0 else 16
+        assert len(names) == 1
+        assert names[0].startswith(f"gemm_bf16_kernel<{m},{max(n, 64) if nn else n},{bk},"), (m, n, k, nn, names)
+
+
+def test_w4a16_cases_run_the_kernels_they_name(host):
+    cases = [c[:4] for c in test_gpu_w4a16_slabs.CASES + test_gpu_w4a16_row_tiles.CASES]
+    r = host(f"""
+out = []
+for m, k, n, group in {[list(c) for c in cases]}:
+    hip.fake_launches()
+    rt.w4a16_gemm(X, B, 5 << 40, 6 << 40, 8, Y, m, k, n, group, t0mi.OUT_F32)
+    out.append([l for l in launches() if l[0].startswith("w4a16")])
+done(out)
+""")
+    after, side, planes = {}, {}, set()
+    for (m, k, n, group), ls in zip(cases, r):
+        for name, _, gy, gz, _ in ls:
+            t = re.fullmatch(r"w4a16_decode_v2<(.*)>", name).group(1).split(",")
+            slabs, tiles = int(t[5]), t[7] == "true"
+            assert int(t[2]) * 32 == group and tiles == (gz > 1)
+            (side if tiles else after).setdefault(group, set()).add(slabs)
+            if gy > 1:
+                planes.add((slabs > 1, tiles))
+    assert after == {32: {3}, 64: {3}, 128: {2, 3, 4}, 256: {1, 2}}
+    assert side == {32: {1, 3}, 64: {1, 2}, 128: {1, 2, 3, 4}, 256: {1, 2}}
+    assert planes == {(True, False), (False, True), (True, True)}
+
+
+def test_f32_cases_run_the_tiles_they_name(host):
+    r = host(f"""
+def kernel(f):
+    hip.fake_launches()
+    f()
+    l = launches()[-1]
+    return l[:2] if l[0].startswith("gemm_f32") else None
+out = []
+for m, n, k in {[list(c) for c in test_gpu_f32_gemm.SHAPES]}:
+    out += [kernel(lambda: rt.matmul(X, B, Y, m, k, n)), kernel(lambda: rt.matmul_backward_data(X, B, Y, m, n, k)),
+            kernel(lambda: rt.matmul_backward_weight(X, B, Y, k, m, n))]
+done([out, [kernel(lambda: rt.matmul_with_wt_bf16(X, B, Y, m, k, n)) + [m, n]
+            for m, n, k in {[list(c) for c in test_gpu_f32_gemm.WT_SHAPES]}]])
+""")
+    products, wt = r
+    seen = {p[0] for p in products if p}
+    tiles = ["32,32", "64,32", "64,64", "128,64", "128,128"]
+    for t in tiles:
+        for mode in ("false,true", "false,false", "true,true"):  # forward, data, weight
+            assert any(s.startswith(f"gemm_f32_kernel<{t},") and s.endswith(f",{mode},false>") for s in seen), (t, mode)
+    got = set()
+    for name, grid, m, n in wt:
+        bm, bn = [int(v) for v in re.match(r"gemm_f32_kernel<(\d+),(\d+),", name).groups()]
+        got.add((bm, grid > -(-m // bm) * -(-n // bn)))
+    assert got == {(32, False), (32, True), (64, False), (64, True)}  # one piece, several
