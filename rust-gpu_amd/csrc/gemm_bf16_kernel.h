@@ -164,16 +164,26 @@ __device__ __forceinline__ void epi_block(float (&v)[4 * Q], const BiasCols<QB>&
   epi_apply(v, b, e);
 }
 
+// With ACC, a block that leaves the accumulator registers here and no earlier.  Vector instructions cannot
+// read those, and the compiler copies every block out of them where the K loop ends unless something ties
+// it to them until its use (128x128x16 on two waves, bf16 output: 134 VGPRs and one wave a SIMD so, 62 and
+// two with ACC).  Not for workgroups of 8 waves, whose sums are in vector registers.
+template <bool ACC>
+__device__ __forceinline__ f32x16 from_acc(f32x16 a) {
+  if constexpr (ACC) asm volatile("" : "+a"(a));
+  return a;
+}
+
 // Stores one 32x32 accumulator block.  Lane l holds rows m (one per lane) and
 // columns n + 8*g + {0..3}, g = 0..3 (n already includes 4*(l >> 5)).  Columns
 // at or beyond N are skipped (the tile's N tail).
 __device__ __forceinline__ void store_block(const GemmParams& p, const f32x16& a, char* ybase, int m, int n,
-                                            bool partial_plane) {
+                                            bool bf16) {
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const int nc = n + g * 8;
     if (nc >= (int)p.N) continue;
-    if (!partial_plane && p.out_bf16) {
+    if (bf16) {
       u32x2 o;
       o.x = pack_bf16x2(a[g * 4 + 0], a[g * 4 + 1]);
       o.y = pack_bf16x2(a[g * 4 + 2], a[g * 4 + 3]);
@@ -199,11 +209,11 @@ __device__ __forceinline__ f32x16 epi_block32(const GemmParams& p, const f32x16&
   return r;
 }
 
-// Stores a wave's FM x FN blocks of 32x32 at (row0, col0): store_block on each, with EPI after the
-// epilogue chain.
-template <int FM, int FN, bool EPI>
+// Stores a wave's FM x FN blocks of 32x32 at (row0, col0), as bf16 or f32: store_block on each, with EPI
+// after the epilogue chain.
+template <int FM, int FN, bool EPI, bool ACC = false>
 __device__ __forceinline__ void store_blocks(const GemmParams& p, const f32x16 (&acc)[FN][FM], char* ybase, int row0,
-                                             int col0, int lane, bool partial_plane) {
+                                             int col0, int lane, bool partial_plane, bool bf16) {
   const int n = col0 + (lane >> 5) * 4;
   BiasCols<EPI ? FN * 4 : 1> bias;
   if constexpr (EPI) bias.load(p, n, 8);
@@ -214,9 +224,9 @@ __device__ __forceinline__ void store_blocks(const GemmParams& p, const f32x16 (
       static_for<FN>([&](auto fnc) {
         constexpr int fn = decltype(fnc)::value;
         if constexpr (EPI)
-          store_block(p, epi_block32(p, acc[fn][fm], bias, fn * 4, partial_plane), ybase, m, n + fn * 32, partial_plane);
+          store_block(p, epi_block32(p, acc[fn][fm], bias, fn * 4, partial_plane), ybase, m, n + fn * 32, bf16);
         else
-          store_block(p, acc[fn][fm], ybase, m, n + fn * 32, partial_plane);
+          store_block(p, from_acc<ACC>(acc[fn][fm]), ybase, m, n + fn * 32, bf16);
       });
     }
   });
@@ -226,10 +236,11 @@ __device__ __forceinline__ void store_tile_direct(const GemmParams& p, const f32
                                                   int row0, int col0, int lane, bool partial_plane) {
   // Stores without a chain get a copy of their own (the bias registers and checks cost split-K planes
   // of 64 x 128 tiles 2 %), except for 256 accumulators a lane, which two copies push into scratch.
+  const bool bf16 = !partial_plane && p.out_bf16;
   if (FM * FN < 16 && (partial_plane || p.epi.n == 0))
-    store_blocks<FM, FN, false>(p, acc, ybase, row0, col0, lane, partial_plane);
+    store_blocks<FM, FN, false>(p, acc, ybase, row0, col0, lane, partial_plane, bf16);
   else
-    store_blocks<FM, FN, true>(p, acc, ybase, row0, col0, lane, partial_plane);
+    store_blocks<FM, FN, true>(p, acc, ybase, row0, col0, lane, partial_plane, bf16);
 }
 
 // swz / swz_nn (the LDS swizzles) and the DMA chunk maps: index_maps.h.
@@ -307,41 +318,19 @@ __device__ __forceinline__ void wait_lgkmcnt0() { __builtin_amdgcn_s_waitcnt(0xF
 // same number of DMA loads (the vmcnt arithmetic below relies on it).
 static __device__ __attribute__((aligned(16))) const uint32_t g_zero16[4] = {0u, 0u, 0u, 0u};
 
-// Stores a wave's FM*32 x FN*32 accumulator block as bf16 through a private
-// LDS block `st` (FM*32 * FN*32 * 2 bytes): each lane writes its 8-byte row
-// pieces with the 16-byte chunks of every row XOR-swizzled by the row index,
-// then the block is read back so that each 16-byte-per-lane store instruction
-// writes 512 / (FN*32) whole rows of FN*64 contiguous bytes (the direct stores
-// of store_block write 16 bytes into each of 32 rows).  The epilogue chain is
-// applied before the conversion.  Caller's contract: a full tile (all rows and
-// columns in range), bf16 output, not a partial plane, 16-byte aligned Y, and
-// no pending LDS reads or DMA into `st`.
-template <int FM, int FN>
-__device__ __forceinline__ void store_tile_bf16_staged(const GemmParams& p, const f32x16 (&acc)[FN][FM], char* st,
-                                                       char* ybase, int row0, int col0, int lane) {
+// Bytes from the start of a staged block (rows of FN*64 bytes) to the 8 bytes of row r, columns
+// fn*32 + gq*8 + 4*(lane >> 5) .. +3.
+template <int FN>
+__device__ __forceinline__ int staged_at(int r, int fn, int gq, int lhalf) {
+  constexpr int CH = FN * 4;  // 16-byte chunks per row
+  return r * FN * 64 + (((fn * 4 + gq) ^ (r & (CH - 1))) * 16) + lhalf * 8;
+}
+// Stores a wave's staged block, whole rows at a time; MASK: rows at or beyond M and columns at or beyond N
+// (a multiple of 8) are skipped.
+template <int FM, int FN, bool MASK>
+__device__ __forceinline__ void store_staged_rows(const GemmParams& p, const char* st, char* ybase, int row0, int col0,
+                                                  int lane) {
   constexpr int TN = FN * 32, CH = TN / 8, RPI = 64 / CH;  // 16-byte chunks per row, rows per store
-  const int lrow = lane & 31, lhalf = lane >> 5;
-  BiasCols<FN * 4> bias;
-  bias.load(p, col0 + lhalf * 4, 8);
-  static_for<FM>([&](auto fmc) {
-    constexpr int fm = decltype(fmc)::value;
-    static_for<FN>([&](auto fnc) {
-      constexpr int fn = decltype(fnc)::value;
-      const int r = fm * 32 + lrow;
-      float v[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = acc[fn][fm][i];
-      if (p.epi.n) epi_block<4>(v, bias, fn * 4, p.epi);
-#pragma unroll
-      for (int gq = 0; gq < 4; ++gq) {
-        const int c = fn * 4 + gq;  // 16-byte chunk of the row
-        u32x2 o;
-        o.x = pack_bf16x2(v[gq * 4], v[gq * 4 + 1]);
-        o.y = pack_bf16x2(v[gq * 4 + 2], v[gq * 4 + 3]);
-        *(u32x2*)(st + r * TN * 2 + ((c ^ (r & (CH - 1))) * 16) + lhalf * 8) = o;
-      }
-    });
-  });
   wait_lgkmcnt0();  // the block is read back only by the wave that wrote it
   const int rr = lane / CH, cc = lane % CH;
   char* yrow = ybase + ((size_t)(row0 + rr) * p.ldy + col0 + cc * 8) * 2;
@@ -350,11 +339,52 @@ __device__ __forceinline__ void store_tile_bf16_staged(const GemmParams& p, cons
     const int r = i * RPI + rr;
     const u32x4 v = *(const u32x4*)(st + r * TN * 2 + ((cc ^ (r & (CH - 1))) * 16));
     u32x4* dst = (u32x4*)(yrow + (size_t)i * RPI * p.ldy * 2);
+    if (MASK && (row0 + r >= (int)p.M || col0 + cc * 8 >= (int)p.N)) continue;
     if (p.stream_out)
       __builtin_nontemporal_store(v, dst);
     else
       *dst = v;
   }
+}
+
+// Stores a wave's FM*32 x FN*32 accumulator block as bf16 through a private
+// LDS block `st` (FM*32 * FN*32 * 2 bytes): each lane writes its 8-byte row
+// pieces with the 16-byte chunks of every row XOR-swizzled by the row index,
+// then the block is read back so that each 16-byte-per-lane store instruction
+// writes 512 / (FN*32) whole rows of FN*64 contiguous bytes (the direct stores
+// of store_block write 16 bytes into each of 32 rows).  With EPI the epilogue chain is
+// applied before the conversion.  Caller's contract: with `full`, all rows and
+// columns in range; bf16 output, not a partial plane, 16-byte aligned Y, and
+// no pending LDS reads or DMA into `st`.
+template <int FM, int FN, bool EPI = true, bool ACC = false>
+__device__ __forceinline__ void store_tile_bf16_staged(const GemmParams& p, const f32x16 (&acc)[FN][FM], char* st,
+                                                       char* ybase, int row0, int col0, int lane, bool full = true) {
+  const int lrow = lane & 31, lhalf = lane >> 5;
+  BiasCols<EPI ? FN * 4 : 1> bias;
+  if constexpr (EPI) bias.load(p, col0 + lhalf * 4, 8);
+  static_for<FM>([&](auto fmc) {
+    constexpr int fm = decltype(fmc)::value;
+    static_for<FN>([&](auto fnc) {
+      constexpr int fn = decltype(fnc)::value;
+      const f32x16 a = from_acc<ACC>(acc[fn][fm]);
+      float v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = a[i];
+      if constexpr (EPI)
+        if (p.epi.n) epi_block<4>(v, bias, fn * 4, p.epi);
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq) {
+        u32x2 o;
+        o.x = pack_bf16x2(v[gq * 4], v[gq * 4 + 1]);
+        o.y = pack_bf16x2(v[gq * 4 + 2], v[gq * 4 + 3]);
+        *(u32x2*)(st + staged_at<FN>(fm * 32 + lrow, fn, gq, lhalf)) = o;
+      }
+    });
+  });
+  if (full)
+    store_staged_rows<FM, FN, false>(p, st, ybase, row0, col0, lane);
+  else
+    store_staged_rows<FM, FN, true>(p, st, ybase, row0, col0, lane);
 }
 
 // Stores one 16x16 accumulator block of v_mfma_f32_16x16x32_bf16: lane l holds
@@ -490,9 +520,9 @@ __device__ __forceinline__ bool exchange_partitions(f32x16 (&acc)[FN][FM], const
 
 // One output tile (tm, tn) of K partition `part`: the whole kernel body, called
 // once by gemm_bf16_kernel and in a loop by the persistent kernel.  SUMS: what becomes of
-// the sums: final or a plane (by p.split_k); a plane always; or the two partitions of a tile summed
-// through `xk` (p.y, p.ldy: the final output).
-enum TileSums { kSumsAny, kSumsPlane, kSumsExchange };
+// the sums: final or a plane (by p.split_k); the same without an epilogue chain, final or a plane in
+// f32 or final in bf16; or the two partitions of a tile summed through `xk` (p.y, p.ldy: the final output).
+enum TileSums { kSumsAny, kSumsF32, kSumsBf16, kSumsExchange };
 template <int BM, int BN, int BK, int WM, int WN, int S, bool NN, TileSums SUMS = kSumsAny>
 __device__ __forceinline__ void gemm_bf16_tile(const GemmParams& p, int tm, int tn, int part,
                                                const XcdExchange* xk = nullptr) {
@@ -836,9 +866,24 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmParams& p, int tm, int 
   // i.e. four consecutive columns per (lane, g): one 16-byte (f32) or
   // 8-byte (bf16) store.  The (fm, fn) loops are expanded at compile time so
   // acc is only ever indexed by constants and stays in registers.
-  if constexpr (SUMS == kSumsPlane) {
+  constexpr bool STAGE = BM * BN <= S * BUF;  // the blocks fit in the LDS ring
+  const bool full = m0 + BM <= (int)p.M && n0 + BN <= (int)p.N;
+  // Without a chain one branch alone reads the accumulators: with two, the compiler copies them (from_acc)
+  // ahead of both.  So bf16 tiles that the matrix cuts are staged as well, and masked on the way from LDS to Y.
+  if constexpr (SUMS == kSumsF32) {
     store_blocks<FM, FN, false>(p, acc, (char*)p.y + (size_t)part * p.y_split_stride, m0 + wm * TM, n0 + wn * TN, lane,
-                                true);
+                                true, false);
+    return;
+  }
+  if constexpr (SUMS == kSumsBf16) {
+    constexpr bool ACC = T::NTHR < 512;
+    if constexpr (STAGE) {
+      __syncthreads();  // every wave has read its last fragments (no DMA is pending)
+      store_tile_bf16_staged<FM, FN, false, ACC>(p, acc, (char*)smem + wave * TM * TN * 2, (char*)p.y, m0 + wm * TM,
+                                                 n0 + wn * TN, lane, full);
+    } else {
+      store_blocks<FM, FN, false, ACC>(p, acc, (char*)p.y, m0 + wm * TM, n0 + wn * TN, lane, false, true);
+    }
     return;
   }
   if constexpr (SUMS == kSumsExchange) {
@@ -849,9 +894,9 @@ __device__ __forceinline__ void gemm_bf16_tile(const GemmParams& p, int tm, int 
   const bool partial_plane = SUMS == kSumsAny && p.split_k > 1;
   char* ybase = (char*)p.y + (partial_plane ? (size_t)part * p.y_split_stride : 0);
   // Full tiles with bf16 output: stage each wave's block through the (now
-  // idle) LDS ring and store whole rows, when the blocks fit in it.
-  if constexpr (BM * BN <= S * BUF) {
-    if (!partial_plane && p.out_bf16 && m0 + BM <= (int)p.M && n0 + BN <= (int)p.N && ((uintptr_t)p.y & 15) == 0) {
+  // idle) LDS ring and store whole rows.
+  if constexpr (STAGE) {
+    if (!partial_plane && p.out_bf16 && full && ((uintptr_t)p.y & 15) == 0) {
       __syncthreads();  // every wave has read its last fragments (no DMA is pending)
       store_tile_bf16_staged<FM, FN>(p, acc, (char*)smem + wave * TM * TN * 2, ybase, m0 + wm * TM,
                                      n0 + wn * TN, lane);
@@ -876,12 +921,12 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_exchange_kernel(GemmPa
   gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, kSumsExchange>(p, tm, tn, part, &xk);
 }
 
-// Split-K planes, without the epilogue's code.
-template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
-__global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_planes_kernel(GemmParams p) {
+// Split-K planes (kSumsF32) and outputs (either) without an epilogue chain, and without the chain's code.
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN, TileSums SUMS>
+__global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_plain_kernel(GemmParams p) {
   int tm, tn, part;
   tile_coords(p, tm, tn, part);
-  gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, kSumsPlane>(p, tm, tn, part);
+  gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, SUMS>(p, tm, tn, part);
 }
 
 }  // namespace t0mi

@@ -177,13 +177,13 @@ __global__ __launch_bounds__(PD_WAVES * 64) void gemm_persistent_decode_kernel(G
 // The generic tile kernel, persistent: work item u (tile, K partition) for u = blockIdx.x,
 // blockIdx.x + gridDim.x, ...; the barrier between items keeps the next item's prologue
 // DMA out of the LDS ring until every wave is done with the previous one.
-template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN, TileSums SUMS>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_bf16_persistent_kernel(GemmParams p) {
   const uint32_t items = p.tiles_m * p.tiles_n * p.split_k;
   for (uint32_t u = blockIdx.x; u < items; u += gridDim.x) {
     int tm, tn, part;
     tile_coords_lin(u, items, p.tiles_m, p.tiles_n, p.xcd_remap, tm, tn, part);
-    gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN>(p, tm, tn, part);
+    gemm_bf16_tile<BM, BN, BK, WM, WN, S, NN, SUMS>(p, tm, tn, part);
     __syncthreads();
   }
 }

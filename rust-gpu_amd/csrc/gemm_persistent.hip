@@ -35,12 +35,22 @@ void launch_decode(const t0mi_ctx* ctx, hipStream_t s, const GemmParams& p) {
   hipLaunchKernelGGL((gemm_persistent_decode_kernel<NN>), dim3(g), dim3(PD_WAVES * 64), 0, s, p);
 }
 
+template <int BM, int BN, int BK, int WM, int WN, int S, bool NN, TileSums SUMS>
+void launch_tile_loop(const t0mi_ctx* ctx, hipStream_t s, const GemmParams& p) {
+  static const uint32_t per_cu = wgs_per_cu(gemm_bf16_persistent_kernel<BM, BN, BK, WM, WN, S, NN, SUMS>, WM * WN * 64);
+  const uint32_t g = persistent_grid(ctx, per_cu, p.tiles_m * p.tiles_n * p.split_k);
+  hipLaunchKernelGGL((gemm_bf16_persistent_kernel<BM, BN, BK, WM, WN, S, NN, SUMS>), dim3(g), dim3(WM * WN * 64), 0, s,
+                     p);
+}
+
 template <int BM, int BN, int BK, int WM, int WN, int S, bool NN>
 void launch_tiles(const t0mi_ctx* ctx, hipStream_t s, const GemmParams& p) {
-  static const uint32_t per_cu = wgs_per_cu(gemm_bf16_persistent_kernel<BM, BN, BK, WM, WN, S, NN>, WM * WN * 64);
-  const uint32_t g = persistent_grid(ctx, per_cu, p.tiles_m * p.tiles_n * p.split_k);
-  hipLaunchKernelGGL((gemm_bf16_persistent_kernel<BM, BN, BK, WM, WN, S, NN>), dim3(g), dim3(WM * WN * 64), 0, s,
-                     p);
+  if (p.epi.n)
+    launch_tile_loop<BM, BN, BK, WM, WN, S, NN, kSumsAny>(ctx, s, p);
+  else if (p.out_bf16)
+    launch_tile_loop<BM, BN, BK, WM, WN, S, NN, kSumsBf16>(ctx, s, p);
+  else
+    launch_tile_loop<BM, BN, BK, WM, WN, S, NN, kSumsF32>(ctx, s, p);
 }
 
 struct PersistentTiles {

@@ -76,7 +76,7 @@ def test_integer_pattern_exact_all_variants(rt, name, layout):
 @pytest.mark.parametrize("name", [v[0] for v in ALL_VARIANTS])
 def test_integer_pattern_bf16_out_all_variants(rt, name, layout):
     """bf16 output: interior tiles take the LDS-staged whole-row store, edge
-    tiles the direct one; both must equal RNE of the exact integer sums."""
+    tiles its masked form; both must equal RNE of the exact integer sums."""
     m, n, k = 520, 264, 128
     cfg = t0mi.preset(name).copy(transpose=layout)
     a, b = int_pattern(m, k, n, layout == t0mi.NN)
@@ -100,6 +100,24 @@ def test_every_prebuilt_kernel_integer_exact(rt, idx):
     y = run_gemm(rt, cfg, a, b, m, n, k)
     ref = oracle.gemm_bf16(a, b, "nn" if cfg.transpose == t0mi.NN else "nt")
     assert np.array_equal(y, ref), f"{cfg.name()}: max diff {np.abs(y - ref).max()}"
+
+
+@pytest.mark.parametrize("idx", range(len(PREBUILT)))
+def test_every_prebuilt_kernel_outputs(rt, idx):
+    """The other outputs of each: bf16 without a chain (a kernel of its own), and bias + ReLU in f32 and
+    bf16; tiles that the matrix cuts in both directions, and whole ones."""
+    cfg = PREBUILT[idx]
+    for m, n, k in [(200, 136, 264), (512, 512, 72)]:
+        a, b = int_pattern(m, k, n, cfg.transpose == t0mi.NN)
+        bias = ((np.arange(n) % 9) - 4).astype(np.float32)
+        ref = oracle.gemm_bf16(a, b, "nn" if cfg.transpose == t0mi.NN else "nt")
+        chain = np.maximum(ref + bias, np.float32(0))
+        relu = cfg.copy(epilogue=t0mi.EPI_BIAS_ADD_RELU)
+        print(f"[prebuilt {idx}] {cfg.name()} {m}x{n}x{k}", flush=True)
+        assert np.array_equal(run_gemm(rt, cfg, a, b, m, n, k, out_bf16=True), oracle.bf16_rne(ref)), cfg.name()
+        assert np.array_equal(run_gemm(rt, relu, a, b, m, n, k, bias=bias), chain), cfg.name()
+        y = run_gemm(rt, relu, a, b, m, n, k, out_bf16=True, bias=bias)
+        assert np.array_equal(y, oracle.bf16_rne(chain)), cfg.name()
 
 
 @pytest.mark.parametrize("layout", [t0mi.NT, t0mi.NN])

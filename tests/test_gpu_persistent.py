@@ -142,6 +142,19 @@ def test_tile_loop_integer_exact(rt, preset, m, n, k, nn):
 
 
 @pytest.mark.parametrize("nn", [0, 1])
+@pytest.mark.parametrize("preset,m,n,k", TILE_CASES)
+def test_tile_loop_without_a_chain(rt, preset, m, n, k, nn):
+    """The loops of kernels without the epilogue's code, f32 and bf16."""
+    spec = spec_of(preset, nn).copy(epilogue=[])
+    a, b = int_pattern(m, k, n, nn, seed=k)
+    ref = oracle.gemm_bf16(a, b, "nn" if nn else "nt")
+    none = np.zeros(1, np.float32)
+    assert np.array_equal(run(rt, spec, a, b, m, n, k, none), ref)
+    assert np.array_equal(run(rt, spec.copy(out_dtype=t0mi.OUT_BF16), a, b, m, n, k, none, out_bf16=True),
+                          oracle.bf16_rne(ref))
+
+
+@pytest.mark.parametrize("nn", [0, 1])
 def test_caller_persistent_spec_without_tile_loop(rt, nn):
     # tile_64x64_k32 made persistent by the caller: the decode kernel at 16 rows, the
     # 64x64 tile's one-shot kernel at 100 rows; both one plane, split-K ignored as the

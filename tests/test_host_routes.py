@@ -11,7 +11,7 @@ import test_gpu_w4a16_row_tiles
 import test_gpu_w4a16_slabs
 from host_runtime import host  # noqa: F401
 
-PLANES = ["gemm_bf16_planes_kernel", "t0mi_splitk_reduce"]
+PLANES = ["gemm_bf16_plain_kernel", "t0mi_splitk_reduce"]
 
 
 @pytest.mark.parametrize("layout", ["NT", "NN"])
@@ -116,7 +116,7 @@ done([before, out])
     assert out["f32"][0][-1] == "gemm_f32_kernel"
     assert out["f32_pieces"][0] == ["cvt_bf16_kernel"] * 2 + out["f32_pieces"][0][2:]
     if limit < 1 << 20:  # no workspace for planes either
-        assert out["tile"][0] == ["gemm_bf16_kernel"]
+        assert out["tile"][0] == ["gemm_bf16_plain_kernel"]
         assert out["w4"][0] == ["w4a16_decode_v2", "t0mi_splitk_reduce"] * 2
     else:
         assert out["gemm"][0] == out["tile"][0] == PLANES
@@ -133,7 +133,7 @@ done([before, out])
 """)
     before, out = r
     assert all(c[1] is None and c[2] == before for c in out.values()), out
-    assert out["f32"][0] == ["gemm_f32_kernel"] and out["tile"][0] == ["gemm_bf16_kernel"]
+    assert out["f32"][0] == ["gemm_f32_kernel"] and out["tile"][0] == ["gemm_bf16_plain_kernel"]
 
 
 @pytest.mark.parametrize("call,warm,then", [
@@ -158,7 +158,7 @@ done([a, b])
 
 
 def test_split_k_planes_run_the_kernel_without_the_epilogue(host):
-    """Every prebuilt tile but single waves of up to 64x64 writes its planes with gemm_bf16_planes_kernel (the
+    """Every prebuilt tile but single waves of up to 64x64 writes its planes with gemm_bf16_plain_kernel (the
     256x256 ping-pong kernel has its own); the chain then runs in the reduce."""
     r = host("""
 import re
@@ -177,8 +177,40 @@ done(out)
     for (bm, bn, bk, wm, wn, st, nn), k in r:
         pingpong = (bm, bn, bk, wm, wn, st) == (256, 256, 64, 2, 4, 2)
         one = wm * wn == 1 and bm * bn <= 64 * 64
-        want = "gemm_bf16_pingpong_kernel" if pingpong else "gemm_bf16_kernel" if one else "gemm_bf16_planes_kernel"
+        want = "gemm_bf16_pingpong_kernel" if pingpong else "gemm_bf16_kernel" if one else "gemm_bf16_plain_kernel"
         assert k == [want, "t0mi_splitk_reduce"], (bm, bn, bk, wm, wn, st, nn)
+
+
+def test_outputs_without_a_chain_run_the_kernels_without_its_code(host):
+    """Every prebuilt tile (but the ping-pong kernel's) and the persistent tile loops: with the epilogue's code
+    and registers a chainless call lost up to half its waves."""
+    r = host("""
+def run(f, *args):
+    f(*args)
+    return [l[0] for l in launches()]
+out = []
+for v in t0mi.variants():
+    for o in (t0mi.OUT_F32, t0mi.OUT_BF16):
+        for e in (t0mi.EPI_STORE_F32, t0mi.EPI_BIAS_ADD_RELU):
+            c = v.copy(out_dtype=o, epilogue=e)
+            out.append([(v.tile_m, v.tile_n, v.tile_k, v.wave_m, v.wave_n) == (256, 256, 64, 2, 4) and v.stages == 0,
+                        o, e, run(rt.gemm, c, X, B, Y, 256, 512, 2048, BIAS)])
+loops = []
+for p in ("tile_persistent_decode", "tile_persistent_128x64_k32", "tile_persistent_256x128_k32"):
+    for o in (t0mi.OUT_F32, t0mi.OUT_BF16):
+        for e in ([], [t0mi.BIAS_ADD]):
+            s = t0mi.tile_preset(p).copy(out_dtype=o, epilogue=e)
+            loops.append([o, bool(e), run(rt.tile_gemm, s, X, B, Y, 256, 512, 2048, BIAS)])
+done([out, loops])
+""")
+    assert len(r[0]) > 240
+    for pingpong, o, e, k in r[0]:
+        want = "gemm_bf16_pingpong_kernel" if pingpong else "gemm_bf16_kernel" if e else "gemm_bf16_plain_kernel"
+        assert len(k) == 1 and k[0].split("<")[0] == want, k
+        assert e or pingpong or k[0].endswith(f",(TileSums){1 + o}>"), k
+    for o, e, k in r[1]:
+        assert len(k) == 1 and k[0].startswith("gemm_bf16_persistent_kernel<"), k
+        assert k[0].endswith(f",(TileSums){0 if e else 1 + o}>"), k
 
 
 @pytest.mark.parametrize("layout", ["NT", "NN"])
@@ -194,7 +226,7 @@ rt.tile_gemm(spec, X, B, Y, 128, 128, 128)
 hip.fake_launches()
 done([run(Y), run(X), run(B), run(X + 128 * 128 * 2 - 16), run(X + 128 * 128 * 2)])
 """)
-    own = f"gemm_bf16_kernel<128,128,32,2,2,2,{str(layout == 'NN').lower()}> 1"
+    own = f"gemm_bf16_plain_kernel<128,128,32,2,2,2,{str(layout == 'NN').lower()},(TileSums)2> 1"
     assert r[0] == r[4] != [own]
     assert r[1] == r[2] == r[3] == [own]
 
@@ -234,7 +266,7 @@ done(out)
     for (m, n, k, nn), names in r:
         bk = 64 if k % 64 == 0 else 32 if k % 32 == 0 else 16
         assert len(names) == 1
-        assert names[0].startswith(f"gemm_bf16_kernel<{m},{max(n, 64) if nn else n},{bk},"), (m, n, k, nn, names)
+        assert names[0].startswith(f"gemm_bf16_plain_kernel<{m},{max(n, 64) if nn else n},{bk},"), (m, n, k, nn, names)
 
 
 def test_w4a16_cases_run_the_kernels_they_name(host):
