@@ -1257,10 +1257,9 @@ static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm
   const bool valid = m && n && k && k % 8 == 0 && n % 8 == 0 && !((x | b | y) & 15) && !(bias & 3) &&
                      !(chain_uses(chain, EOP_BIAS) && !bias);
   if (tile_split_k(s) == 1 && valid && !output_meets_operands(cfg, x, b, y, m, n, k, n)) {
-    if (cfg.transpose == T0MI_NT) {
-      const int rc = run_gemm_decode_nt(ctx, x, b, y, m, n, k, cfg.out_dtype, bias, chain);
-      if (rc <= 0) return rc;
-    }
+    // NT calls of up to 16 rows as well: not run_gemm_auto, whose one-launch decode kernel has a long fixed
+    // time here (9 x 2584 x 320: 4.3 us on the spec's tile, 9.2 by that kernel, 4.3 by the schedule; 16 x 240
+    // x 4736: 27.0, 29.2, 6.7; 249 random calls: the schedule 0.63 of the spec's tile, the kernel 0.83).
     AutoPlan pl;
     if (cached_auto_plan(m, n, k, cfg.transpose, cfg.out_dtype, (uint32_t)ctx->cu_count, &pl)) {
       bool ok = false;

@@ -181,6 +181,17 @@ done(out)
         assert k == [want, "t0mi_splitk_reduce"], (bm, bn, bk, wm, wn, st, nn)
 
 
+@pytest.mark.parametrize("m,n,k", [(9, 2584, 320), (16, 240, 4736), (1, 4096, 512)])
+def test_tile_spec_of_few_rows_runs_the_schedule(host, m, n, k):
+    """NT of up to 16 rows: the ranked schedule, not the decode kernel that run_gemm_auto has for them."""
+    r = host(f"""
+spec = t0mi.tile_preset("tile_64x64_k16")
+rt.tile_gemm(spec, X, B, Y, {m}, {n}, {k})  # buffers are made
+done(names(rt.tile_gemm, spec, X, B, Y, {m}, {n}, {k}))
+""")
+    assert r and all(x in ("gemm_bf16_plain_kernel", "gemm_bf16_exchange_kernel", "t0mi_splitk_reduce") for x in r), r
+
+
 def test_outputs_without_a_chain_run_the_kernels_without_its_code(host):
     """Every prebuilt tile (but the ping-pong kernel's) and the persistent tile loops: with the epilogue's code
     and registers a chainless call lost up to half its waves."""
