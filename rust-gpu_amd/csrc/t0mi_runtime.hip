@@ -1243,13 +1243,23 @@ extern "C" int t0mi_auto_gemm_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t 
 
 // ------------------------------------------------------------ tile_ir GEMM ----
 
+// Products so short that what a workgroup stores takes longer than what it multiplies: the ranking leaves
+// the stores of a CU out and picks tiles of 128 and 256 rows, too few to fill the chip, there.  Of 1800
+// random calls through specs (m to 4096, n to 8192, k to 588), time by the ranked schedule over that on the
+// spec's own tile: 256 rows, K up to 32 1.82 (1527 x 672 x 32: 4.1 -> 10.6 us), 40 to 128 1.12, 136 to 160
+// 0.87 (4 of 10 slower, by up to 1.45), above 0.74; 128 rows, K of 40 to 64 0.92 (10 of 25 slower, by up to
+// 1.23), above 0.83.
+static bool short_for_ranked_tile(const AutoPlan& pl, uint32_t k) {
+  return k <= (pl.head.tile_m >= 256 ? 160u : pl.head.tile_m >= 128 ? 64u : 0u);
+}
+
 // Y = epi(X . B) of a one-shot spec into one plane.  A spec without split-K leaves the schedule
 // open, and its tile is one of an RDNA part's (64 x 64 x 16 on one wave, say), so the schedule that
 // auto_select ranks first for the shape runs under the spec's name, kernargs and grid, as for the
 // persistent presets (1000 x 2752 x 2056 NT, bias + GELU, bf16 out, tile_auto_select's 64x64 k16: 63.8
 // us on its own tile, 24.1 so).  The spec's tile remains for specs that name their split-K, where Y
 // lies over X or B (one tile, the whole of Y, is stored after its operands are read; the schedule may
-// cut it into several), for calls whose arguments are refused (it reports them), and where the schedule's split-K planes would
+// cut it into several), for short K (short_for_ranked_tile), for calls whose arguments are refused (it reports them), and where the schedule's split-K planes would
 // need workspace that cannot be had now (a capture, live graphs holding its address, no memory left).
 static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm_config& cfg, const GemmLaunchEntry* e,
                          uint64_t x, uint64_t b, uint64_t y, uint64_t bias, uint32_t m, uint32_t n, uint32_t k,
@@ -1261,7 +1271,8 @@ static int run_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec& s, const t0mi_gemm
     // time here (9 x 2584 x 320: 4.3 us on the spec's tile, 9.2 by that kernel, 4.3 by the schedule; 16 x 240
     // x 4736: 27.0, 29.2, 6.7; 249 random calls: the schedule 0.63 of the spec's tile, the kernel 0.83).
     AutoPlan pl;
-    if (cached_auto_plan(m, n, k, cfg.transpose, cfg.out_dtype, (uint32_t)ctx->cu_count, &pl)) {
+    if (cached_auto_plan(m, n, k, cfg.transpose, cfg.out_dtype, (uint32_t)ctx->cu_count, &pl) &&
+        !short_for_ranked_tile(pl, k)) {
       bool ok = false;
       if (int rc = try_workspace(ctx, plan_workspace(pl, m, n), &ok)) return rc;
       if (ok) return run_gemm_planned(ctx, pl, cfg.transpose, x, b, y, m, n, k, cfg.out_dtype, bias, &chain);

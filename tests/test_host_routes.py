@@ -192,6 +192,25 @@ done(names(rt.tile_gemm, spec, X, B, Y, {m}, {n}, {k}))
     assert r and all(x in ("gemm_bf16_plain_kernel", "gemm_bf16_exchange_kernel", "t0mi_splitk_reduce") for x in r), r
 
 
+def test_tile_spec_keeps_its_tile_for_short_k(host):
+    """Short K, where the ranking picks tiles of 128 and 256 rows, too few to fill the chip."""
+    r = host("""
+spec = t0mi.tile_preset("tile_64x64_k16")
+out = []
+for m, n, k, nn in [(1527, 672, 32, 1), (277, 4240, 16, 1), (1998, 2432, 136, 1), (2314, 1736, 200, 1),
+                    (321, 2896, 48, 1), (1423, 1760, 88, 1), (100, 1000, 40, 1)]:
+    head = t0mi.auto_gemm_plan(m, n, k, nn, t0mi.OUT_F32)[0]
+    hip.fake_launches()
+    rt.tile_gemm(spec.copy(transpose=nn), X, B, Y, m, n, k)
+    out.append([head.tile_m, k, [l[0] for l in launches() if "fill" not in l[0]]])
+done(out)
+""")
+    assert [x[0] for x in r] == [256, 256, 256, 256, 128, 128, 64], r
+    for tile_m, k, names in r:
+        own = k <= {256: 160, 128: 64}.get(tile_m, 0)
+        assert (names[0].split("<")[1].split(",")[:3] == ["64", "64", "16"]) == own, (tile_m, k, names)
+
+
 def test_outputs_without_a_chain_run_the_kernels_without_its_code(host):
     """Every prebuilt tile (but the ping-pong kernel's) and the persistent tile loops: with the epilogue's code
     and registers a chainless call lost up to half its waves."""
