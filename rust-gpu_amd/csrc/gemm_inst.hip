@@ -30,8 +30,10 @@ static void launch_variant(dim3 g, hipStream_t s, const GemmParams& p) {
   // 128x4096x4096 NN in 4, 64x128x64: 14.0-14.3 and 13.9.  Planes of single waves of up to 64x64 keep the
   // one kernel: with more of them on a SIMD they run 4-6 % slower (2048x4096x1024 in 2 parts, 32x64x16 NN
   // 62.1 and 66.1 us, 64x64x16 NT 67.2 and 70.5).
-  if (p.split_k > 1 ? WM * WN > 1 || BM * BN > 64 * 64 : p.epi.n == 0) {
-    if (p.split_k > 1 || !p.out_bf16)
+  // The bf16 one stores 16 bytes at a time; a raw dispatch may bring a Y of less alignment.
+  const bool planes = p.split_k > 1, aligned = !p.out_bf16 || ((uintptr_t)p.y & 15) == 0;
+  if (planes ? WM * WN > 1 || BM * BN > 64 * 64 : p.epi.n == 0 && aligned) {
+    if (planes || !p.out_bf16)
       hipLaunchKernelGGL((gemm_bf16_plain_kernel<BM, BN, BK, WM, WN, S, NN, kSumsF32>), g, dim3(WM * WN * 64), 0, s, p);
     else
       hipLaunchKernelGGL((gemm_bf16_plain_kernel<BM, BN, BK, WM, WN, S, NN, kSumsBf16>), g, dim3(WM * WN * 64), 0, s, p);

@@ -181,6 +181,22 @@ done(out)
         assert k == [want, "t0mi_splitk_reduce"], (bm, bn, bk, wm, wn, st, nn)
 
 
+def test_dispatch_with_y_of_less_alignment(host):
+    """A raw dispatch does not ask for a Y aligned to 16 bytes: bf16 there takes the kernel that asks itself."""
+    r = host("""
+out = []
+for o in (t0mi.OUT_F32, t0mi.OUT_BF16):
+    c = t0mi.preset("tile_128x64_k32").copy(out_dtype=o)
+    for y in (Y, Y + 8):
+        hip.fake_launches()
+        rt.dispatch(rt.kernel(c), t0mi.compute_grid_auto(c, 256, 128), t0mi.build_kernargs(X, B, y, 64, 128, 256, c), False)
+        out.append([l[0].split("<")[0] for l in launches()])
+done(out)
+""")
+    plain, both = ["gemm_bf16_plain_kernel"], ["gemm_bf16_kernel"]
+    assert r == [plain, plain, plain, both]
+
+
 @pytest.mark.parametrize("m,n,k", [(9, 2584, 320), (16, 240, 4736), (1, 4096, 512)])
 def test_tile_spec_of_few_rows_runs_the_schedule(host, m, n, k):
     """NT of up to 16 rows: the ranked schedule, not the decode kernel that run_gemm_auto has for them."""
