@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the gfx950 GEMM hot path (one MI355X).
 
-Headline (BASELINE.json metric): bf16 GEMM TFLOPS at 4096^3 (config 2: NN layout,
+Headline: bf16 GEMM TFLOPS at 4096^3 (config 2: NN layout,
 N(0,1) inputs, fp32 accumulate, bf16 output) as a fraction of the dense bf16
 MFMA peak, plus the W4A16 decode GEMM (config 4: M=16, K=4096, N=11008, int4
 weights, group 128, zero point 8, bf16 out) in HBM GB/s against the HBM peak.

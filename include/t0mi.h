@@ -412,7 +412,15 @@ int t0mi_tile_compute_grid(const t0mi_tile_spec* s, uint32_t m, uint32_t n, uint
  * (tile_ir.rs:887; compile.rs:1398): looks up the prebuilt gfx950 kernel with
  * the spec's tile_m x tile_n x tile_k, or the one covering it (tile_k 48 as
  * three 16-K steps; NN tiles narrower than 64 columns on the 64-column NN
- * kernel).  The handle dispatches with the spec's own kernarg layout and grid;
+ * kernel).  That kernel runs when the spec names its split-K; a spec without
+ * split-K (and not persistent) leaves the schedule open, and a call of it runs
+ * the schedule t0mi_auto_gemm_plan ranks first for its sizes, whose split-K
+ * planes the library's workspace then holds (it may grow on the first call of a
+ * size, which waits for the stream).  The spec's own kernel remains for short K
+ * where that schedule has large tiles, where Y lies over X or B, and where the
+ * workspace cannot grow (in a capture, while graphs are alive, out of memory);
+ * the two sum in another order.  The handle dispatches with the spec's own
+ * kernarg layout and grid;
  * M comes from the kernarg (0 = derive it from the grid, padded as gemm_gen
  * does).  A persistent spec (one workgroup looping over the tiles in the
  * reference, tile_ir.rs:540-604, 1062-1120) runs as one launch of a persistent
@@ -427,7 +435,8 @@ int t0mi_tile_kernel_get(t0mi_ctx* ctx, const t0mi_tile_spec* s, t0mi_kernel** o
 /* One-call tile GEMM: Y[m,n] = epilogue(X[m,k] . B) for the spec's transpose,
  * with the chain's arguments; split_k > 1 is reduced deterministically (the
  * reference's tile_ir split-K writes every partition to one plane,
- * tile_ir.rs:4577-4581; here the sum is correct).  A persistent spec takes the
+ * tile_ir.rs:4577-4581; here the sum is correct).  Without split-K the kernel
+ * is chosen as at t0mi_tile_kernel_get.  A persistent spec takes the
  * persistent kernels described at t0mi_tile_kernel_get.  Asynchronous. */
 int t0mi_tile_gemm(t0mi_ctx* ctx, const t0mi_tile_spec* s, uint64_t x, uint64_t wt, uint64_t y, uint32_t m,
                    uint32_t n, uint32_t k, uint64_t bias, float scale, float clamp_min, float clamp_max);
@@ -559,10 +568,16 @@ int t0mi_gptq_convert(t0mi_ctx* ctx, uint64_t packed, uint64_t scales_f32, uint6
 /* ---- Ignis matmul caller (src/ignis/ops/bf16_matmul.rs:33-423) ------------- */
 /* The reference converts f32 -> bf16 on the host (round to nearest even,
  * bf16_matmul.rs:372), transposes W, pads every dimension to tile multiples,
- * runs the NT gemm_gen kernel with f32 output and unpads.  Here the conversion
- * (and, where a GEMM operand needs it, the transpose) runs on the GPU into a
- * library-owned buffer, NN is native and ragged shapes need no padding.  All
- * buffers are device f32, row-major, and the calls are asynchronous. */
+ * runs the NT gemm_gen kernel with f32 output and unpads.  Here small and
+ * mid-sized products run as one launch on the f32 operands, which are rounded
+ * to bf16 on the way into LDS; for large ones, and where the output lies over
+ * an operand, the conversion (and, where a GEMM operand needs it, the
+ * transpose) runs on the GPU into a library-owned buffer.  NN is native and
+ * ragged shapes need no padding.  The first product makes 40 MiB of exchange
+ * slots for the one-launch route, and that route also holds the conversion
+ * buffer and workspace of the other one for its sizes, both as far as memory
+ * allows.  All buffers are device f32, row-major, and the calls are
+ * asynchronous. */
 
 /* f32 -> bf16 round-to-nearest-even of `count` elements (bf16_matmul.rs:372). */
 int t0mi_f32_to_bf16(t0mi_ctx* ctx, uint64_t src_f32, uint64_t dst_bf16, uint64_t count);

@@ -22,7 +22,7 @@
 //        per row, fragments read with ds_read_b128.
 //   NT: B = WT[N,K] row-major (ldb = K) — the reference's only implemented layout;
 //        LDS tile [BN][BK] like A.
-//   NN: B = B[K,N] row-major (ldb = N) — BASELINE.json's layout.  The LDS tile is
+//   NN: B = B[K,N] row-major (ldb = N) — the benchmark's layout.  The LDS tile is
 //        stored as loaded, [BK][BN], and the K-contiguous MFMA operand is formed
 //        by ds_read_b64_tr_b16 (gfx950 transpose read): within a 16-lane group,
 //        lane l receives element (l % 4) of the 8-byte chunks addressed by lanes

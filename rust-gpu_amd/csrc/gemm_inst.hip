@@ -25,8 +25,8 @@ static void launch_variant(dim3 g, hipStream_t s, const GemmParams& p) {
   }
   // Split-K's planes and outputs without an epilogue chain: kernels without its code, whose chain and biases
   // take up to twice the registers of the rest (128x128x16 on two waves: 62 VGPRs and two waves a SIMD, 234
-  // and one with it).  4096x4096x512 NN, f32 out, 128x128x16: 41.0 us with the code in the kernel, 30.8
-  // without; bf16 out, 128x256x32: 34.1 and 26.5; 2048x4096x1024 NN in 2 parts, 128x128x16: 55.1 and 44.2;
+  // and one with it).  4096x4096x512 NN, f32 out, 128x128x16: 41.0 us with the code in the kernel, 30.4
+  // without; bf16 out, 128x256x32: 34.1 and 27.4; 2048x4096x1024 NN in 2 parts, 128x128x16: 55.1 and 44.2;
   // 128x4096x4096 NN in 4, 64x128x64: 14.0-14.3 and 13.9.  Planes of single waves of up to 64x64 keep the
   // one kernel: with more of them on a SIMD they run 4-6 % slower (2048x4096x1024 in 2 parts, 32x64x16 NN
   // 62.1 and 66.1 us, 64x64x16 NT 67.2 and 70.5).

@@ -5,7 +5,7 @@
 // <256, 256, 64, 2, 4, 2, NN> (so results are bit-identical to it); it replaces
 // that instantiation where its preconditions hold (pingpong_ok below):
 //   src/t0/gemm_gen.rs:668-1438 (generate_lds_db): NT is the reference's
-//   layout, NN the one BASELINE.json names.
+//   layout, NN the benchmark's.
 //
 // Schedule.  Waves 0-3 (group 0) own rows 0-127 of the tile and waves 4-7
 // (group 1) rows 128-255; wave w and wave w+4 run on the same SIMD.  Every

@@ -361,9 +361,10 @@ static uint32_t decode_max_slabs(uint32_t group) { return group == 256 ? 2 : gro
 // Row tiles of the decode kernel: slabs per workgroup, with the tiles of a call either in one
 // launch (grid.z) or one launch after another.  A workgroup takes about 4.9 + 2.5 us per slab (K =
 // 4096: its activations, at 50 GB/s per CU) and a CU runs one at a time, so one launch costs its
-// rounds of workgroups and pays where the strips leave CUs idle: N = 4096 (64 strips), 100 rows, 27.3
-// -> 10.5 us with four tiles of 2 slabs; 191 rows 44.8 -> 14.1 us with four of 3; 17 rows 9.2 -> 7.4
-// us with two of 1; N = 1376, 191 rows 45.4 -> 11.7 us.  At N = 11008 (172 strips) the tiles of one
+// rounds of workgroups and pays where the strips leave CUs idle: N = 4096 (64 strips), 100 rows, 26.0
+// -> 9.9 us with four tiles of 2 slabs; 191 rows 43.8 -> 12.4 us with four of 3; 17 rows 8.7 -> 6.4
+// us with two of 1; N = 1376, 191 rows 42.9 -> 9.4 us.  For K from 256 to 3072 too (150 random calls of
+// 17 to 191 rows: none slower than one launch after another, 0.53 of its time, geometric mean).  At N = 11008 (172 strips) the tiles of one
 // launch run in two or three rounds (28.9 us at 100 rows) where a launch of 4 slabs and one of 3
 // follow each other on idle CUs (28.4).  Returns the slabs per workgroup of one launch, or 0 for
 // one launch after another.

@@ -1,6 +1,6 @@
 """GPU parity tests of the bf16 GEMM (HIP kernels through the C ABI) against the CPU oracle.
 
-Bars (BASELINE.json north_star):
+Bars:
   - integer-valued inputs: bit-exact (every partial sum is an exactly
     representable integer, so any summation order gives the same result);
   - random inputs: max|err| <= 1e-2 * sqrt(K) * max|a| * max|b|, relative
